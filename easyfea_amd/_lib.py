@@ -13,6 +13,21 @@ LIB_PATH = os.path.join(_HERE, "libefea_hip.so")
 vp = C.c_void_p
 i32, i64, f64, sz = C.c_int, C.c_int64, C.c_double, C.c_size_t
 
+
+
+class ResidentPlan(C.Structure):
+    """``efea_resident_plan`` of ``include/efea.h``."""
+
+    _fields_ = ([(n, C.c_int32) for n in ("dof_n", "slots", "passes", "nblk", "max_halo", "nex", "nagg", "npiece",
+                                          "max_pieces", "ncollect")]
+                + [(n, vp) for n in ("rows", "lidx", "halo_ptr", "halo_ex", "pub", "pub_ptr", "pub_pos", "self",
+                                     "piece_ptr", "piece_agg", "piece_chunk",
+                                     "chunk_piece", "collect")])
+
+
+_plan = C.POINTER(ResidentPlan)
+_resident = [_plan, i32, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, sz, f64, f64, i32, i32, f64, vp]
+
 # name -> (restype, argtypes)
 SIGNATURES = {
     "efea_version": (i32, []),
@@ -90,6 +105,12 @@ SIGNATURES = {
         [i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, vp, i32, i32, vp, vp, i32, vp, vp, vp,
          vp, sz, f64, f64, i32, i32, i32, vp, vp, vp],
     ),
+    "efea_resident_shape": (i32, [i32, i32, i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
+    "efea_resident_fits": (i32, [_plan]),
+    "efea_resident_workspace_bytes": (sz, [i32, _plan]),
+    "efea_solve_resident": (i32, _resident + [vp]),
+    "efea_resident_start": (i32, _resident),
+    "efea_resident_finish": (i32, _resident + [vp, vp]),
     "efea_batch_create": (i32, [i32, i32, i32, i32, i32, C.POINTER(vp)]),
     "efea_batch_destroy": (i32, [vp]),
     "efea_batch_add": (

@@ -9,6 +9,7 @@
 
 #include "efea_common.h"
 #include "pcg_device.h"
+#include "resident.h"
 
 namespace efea {
 
@@ -575,6 +576,94 @@ int efea_pcg2p_finish(PCG2P_PARAMS, double* info, int* resumed) {
 #undef PCG2P_RUN
 #undef PCG2P_CHECK
 #undef PCG2P_PARAMS
+
+int efea_resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, int* slots, int* passes) {
+  if (!lanes || !slots || !passes) {
+    set_error("efea_resident_shape: null pointer");
+    return EFEA_ERR_ARG;
+  }
+  return resident_shape(dof_n, max_neighbours, min_passes, lanes, slots, passes);
+}
+
+int efea_resident_fits(const efea_resident_plan* plan) { return plan ? resident_fits(*plan) : 0; }
+
+size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan) {
+  return plan ? resident_workspace_bytes(Nnode, plan->dof_n, *plan) : 0;
+}
+
+// Argument checks shared by efea_solve_resident and its deferred form.
+static int resident_check(const char* fn, const efea_resident_plan* P, int Nnode, const int32_t* node_ptr,
+                          const double* values64, const double* Minv, const double* rel, const double* Ainv, int ld,
+                          const double* b, double* x, void* workspace, size_t workspace_bytes, int maxit) {
+  if (!P || Nnode <= 0 || !node_ptr || !values64 || !Minv || !b || !x || !workspace || !P->rows || !P->lidx ||
+      !P->halo_ptr || !P->halo_ex || !P->pub || !P->pub_ptr || !P->pub_pos || !P->self) {
+    set_error("%s: null pointer or empty system", fn);
+    return EFEA_ERR_ARG;
+  }
+  if (P->nblk <= 0 || P->max_halo < 0 || P->nex < 0 || P->nagg < 0 || maxit < 1 || !resident_fits(*P)) {
+    set_error("%s: no kernel for this plan (dof_n %d, slots %d, passes %d, %d blocks)", fn, P->dof_n, P->slots,
+              P->passes, P->nblk);
+    return EFEA_ERR_ARG;
+  }
+  if (P->nagg > 0 && (P->dof_n < 2 || P->npiece <= 0 || P->max_pieces <= 0 || !P->piece_ptr || !P->piece_agg ||
+                      !P->piece_chunk || !P->chunk_piece || !P->collect || !rel || !Ainv ||
+                      ld < coarse_ld(P->nagg, P->dof_n))) {
+    set_error("%s: incomplete coarse space", fn);
+    return EFEA_ERR_ARG;
+  }
+  if (workspace_bytes < resident_workspace_bytes(Nnode, P->dof_n, *P)) {
+    set_error("%s: workspace of %zu bytes, %zu needed", fn, workspace_bytes,
+              resident_workspace_bytes(Nnode, P->dof_n, *P));
+    return EFEA_ERR_SIZE;
+  }
+  return EFEA_OK;
+}
+
+#define RESIDENT_PARAMS                                                                                           \
+  const efea_resident_plan *plan, int Nnode, const int32_t *node_ptr, const double *values64,                     \
+      const uint8_t *known, const double *Minv, const double *rel, const double *Ainv, int ld, const double *b,   \
+      double *x, void *workspace, size_t workspace_bytes, double tol_residual, double tol_anorm, int maxit,       \
+      int first_check, double wait_ms, void *stream
+#define RESIDENT_CHECK(fn)                                                                                        \
+  resident_check(fn, plan, Nnode, node_ptr, values64, Minv, rel, Ainv, ld, b, x, workspace, workspace_bytes, maxit)
+#define RESIDENT_RUN(info, phase, resumed)                                                                        \
+  solve_resident(*plan, Nnode, node_ptr, values64, known, Minv, rel, Ainv, ld, b, x, workspace, tol_residual,     \
+                 tol_anorm, maxit, first_check, wait_ms, STREAM(stream), info, phase, resumed)
+
+int efea_solve_resident(RESIDENT_PARAMS, double* info) {
+  if (!info) {
+    set_error("efea_solve_resident: null info");
+    return EFEA_ERR_ARG;
+  }
+  if (int e = RESIDENT_CHECK("efea_solve_resident")) return e;
+  return RESIDENT_RUN(info, PCGP_WHOLE, nullptr);
+}
+
+int efea_resident_start(RESIDENT_PARAMS) {
+  if (int e = RESIDENT_CHECK("efea_resident_start")) return e;
+  if (first_check < 1) {
+    set_error("efea_resident_start: first_check %d (the iterations to queue, >= 1)", first_check);
+    return EFEA_ERR_ARG;
+  }
+  return RESIDENT_RUN(nullptr, PCGP_START, nullptr);
+}
+
+int efea_resident_finish(RESIDENT_PARAMS, double* info, int* resumed) {
+  if (!info) {
+    set_error("efea_resident_finish: null info");
+    return EFEA_ERR_ARG;
+  }
+  if (int e = RESIDENT_CHECK("efea_resident_finish")) return e;
+  if (first_check < 1) {
+    set_error("efea_resident_finish: first_check %d (the start's, >= 1)", first_check);
+    return EFEA_ERR_ARG;
+  }
+  return RESIDENT_RUN(info, PCGP_FINISH, resumed);
+}
+
+#undef RESIDENT_RUN
+#undef RESIDENT_CHECK
+#undef RESIDENT_PARAMS
 
 int efea_batch_create(int mode, int dof_n, int group, int two_level, int capacity, void** handle) {
   if (!handle) {

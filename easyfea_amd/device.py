@@ -20,6 +20,7 @@ from ._utils import ElemType, MatrixType
 from .assembly_map import CsrMap, VecMap, build_csr_map, build_vec_map
 from .coarse import aggregate, coarse_pairs, default_target, n_modes
 from .quadrature import N_pg, dN_pg, gauss_points
+from .resident import Resident
 
 
 def require_gpu() -> torch.device:
@@ -218,6 +219,14 @@ class CsrPattern:
         self.group = _lib.load().efea_default_group(cmap.dof_n, cmap.max_neighbours, cmap.Nn)
         nd = cmap.nPe * cmap.dof_n
         self.n_entries = Ne * nd * nd
+
+    def resident(self, cs: Optional["CoarseSpace"] = None) -> Optional[Resident]:
+        """The plan of this pattern's resident solves (block Jacobi, or two-level
+        with ``cs``), built on first use; None if no kernel takes it."""
+        c = self.__dict__.setdefault("_resident", {}) if cs is None else cs.__dict__.setdefault("_resident", {})
+        if "plan" not in c:
+            c["plan"] = Resident.build(self, cs)
+        return c["plan"]
 
     def coarse(self, target: Optional[int] = None) -> "CoarseSpace":
         target = default_target(self.dim) if target is None else int(target)
@@ -459,8 +468,11 @@ class SolveInfo:
     precond: str = "bj"
     coarse_reused: bool = False
     refine: bool = False  # FP32 inner PCG inside FP64 iterative refinement
-    pipelined: bool = False  # pipelined PCG (block Jacobi: one launch per iteration; two-level: two)
+    # taken for a latency-bound solve: the pipelined PCG (block Jacobi: one launch per iteration;
+    # two-level: two), or resident in its place
+    pipelined: bool = False
     isolated: int = 0  # nodes given aggregates of their own after a stalled solve
+    resident: bool = False  # the whole solve in one launch (efea_solve_resident)
 
 
 # Mixed-precision strategies of a single two-level solve:
@@ -489,6 +501,9 @@ PIPELINE_MAX_COARSE = 4096
 # stopped 5e-9 to 6e-8 from the direct solution depending on the
 # replacement period, against 3e-10 for the classic iteration.
 PIPELINE_BJ_MAX_EXPECTED = 128
+# Longest wait of a resident solve's block for another one before the solve is
+# given up and redone with the classic iteration (0: the library's 250 ms).
+RESIDENT_WAIT_MS = 0.0
 # A phase-field displacement solve that stalls with fully damaged nodes is
 # redone with those nodes as singleton aggregates; the attempts before stop
 # after this many iterations (or 4x the previous solve's), the coarse space
@@ -569,6 +584,8 @@ class SolveJob:
         self.method = "pcg"
         self.pipe_replace_every = 0  # pipelined block Jacobi: residual replacement period (0: the library's)
         self.pipelined = False  # decided by run(), as refine
+        # plan of a solve in one launch, its matrix in registers (decided with pipelined)
+        self.resident: Optional[Resident] = None
         # defer: the single-system driver may start the solve without waiting
         # for it (start(): a PendingSolve the owner finishes later)
         self.defer = False
@@ -631,14 +648,24 @@ class SolveJob:
         return SolveInfo(int(raw[0]), float(raw[1]), int(raw[2]), int(raw[3]),
                          "fp64" if self.precision == 64 else "mixed", self.fallback, self.precond,
                          self.coarse_reused, self.refine and self.precision == 32,
-                         self.pipelined, self.n_isolated)
+                         self.pipelined, self.n_isolated, self.resident is not None)
+
+    def _wants_resident(self) -> Optional[Resident]:
+        """The plan of a resident solve: FP64, unless the caller asked for the
+        classic iteration, whatever the expected count (its recurrences do not
+        drift), wherever the matrix fits the chip's registers."""
+        if self.pipelined_mode is False or self.precision != 64 or self.method != "pcg":
+            return None
+        if self.precond == "two-level":
+            return self.A.pattern.resident(self.A.coarse(self.coarse_target))
+        return self.A.pattern.resident()
 
     def _wants_pipeline(self) -> bool:
         if self.pipelined_mode is False or self._wants_refine():
             return False
         if self.precond == "bj":
             # one launch per iteration; its grid covers the node groups in one pass
-            if self.A.Nn * self.A.group > _lib.load().efea_pcgp_max_lanes():
+            if self.resident is None and self.A.Nn * self.A.group > _lib.load().efea_pcgp_max_lanes():
                 return False
             if self.pipelined_mode is True:
                 return True
@@ -646,6 +673,8 @@ class SolveJob:
             return n is not None and n <= PIPELINE_BJ_MAX_EXPECTED and self.A.nnz * 8 < REFINE_MIN_MATRIX_BYTES
         if self.precond != "two-level":
             return False
+        if self.resident is not None:
+            return True
         cs = self.A.coarse(self.coarse_target)
         if cs.nagg * cs.nm > PIPELINE_MAX_COARSE or cs.pipeline(self.A.pattern, self.A.group).nchunk > 1024:
             return False
@@ -706,9 +735,23 @@ class SolveJob:
                 ptr(self.x), ptr(buf), nbytes, self.tol_residual, self.tol_anorm, self.maxit, check_every,
                 first_check)
 
+    def _resident_args(self, ws: Workspace, first_check: int) -> tuple:
+        """The arguments of ``efea_solve_resident`` (and of its deferred form)
+        before the stream."""
+        A, cs, r = self.A, self.cs, self.resident
+        buf = ws.get(r.nbytes)
+        two = self.precond == "two-level"
+        return (C.byref(r.plan), A.Nn, ptr(A.node_ptr), ptr(A.values), ptr(self.known), ptr(self.Minv),
+                ptr(cs.rel) if two else None, ptr(self.Ainv) if two else None, cs.ld if two else 0, ptr(self.b),
+                ptr(self.x), ptr(buf), r.nbytes, self.tol_residual, self.tol_anorm, self.maxit, first_check,
+                RESIDENT_WAIT_MS)
+
     def _solve_once(self, ws: Workspace):
         A = self.A
         raw = (C.c_double * 4)()
+        if self.resident is not None:
+            rc = _lib.call("efea_solve_resident", *self._resident_args(ws, 0), stream_ptr(), C.cast(raw, C.c_void_p))
+            return rc, self.info(raw)
         check_every, first_check = self._polls()
         v32 = A.values32 if self.precision == 32 else None
         c32 = A.corr32 if self.precision == 32 else None
@@ -775,9 +818,10 @@ class SolveJob:
 
     def _prepare(self) -> None:
         self.refine = self._wants_refine()
+        self.resident = self._wants_resident()
         self.pipelined = self._wants_pipeline()
         isolating = self.isolate is not None and self.A.pattern.coord is not None
-        if (self.pipelined or isolating) and self.x0 is None:
+        if (self.pipelined or self.resident is not None or isolating) and self.x0 is None:
             self.x0 = self.x.clone()
         self._maxit = self.maxit
         if isolating:
@@ -787,12 +831,12 @@ class SolveJob:
     def _conclude(self, ws: Workspace, rc: int, si: SolveInfo, raise_on_fail: bool) -> SolveInfo:
         """The fallbacks of a solve that did not converge (see ``run``)."""
         isolating = self.isolate is not None and self.A.pattern.coord is not None
-        if rc != 0 and self.pipelined:
-            # a pipelined breakdown (rounding in its recurrences): the classic
-            # iteration from the same start
+        if rc != 0 and (self.pipelined or self.resident is not None):
+            # a pipelined breakdown (rounding in its recurrences) or a resident
+            # solve given up: the classic iteration from the same start
             self.pipeline_failure = (rc, _lib.last_error(), si)
             self.x.copy_(self.x0)
-            self.pipelined = False
+            self.pipelined, self.resident = False, None
             self.fallback = True
             rc, si = self._solve_once(ws)
         if rc != 0 and self.precision == 32:
@@ -815,7 +859,8 @@ class SolveJob:
         if self.method != "pcg" or not self.expected_iterations:
             return None
         self.refine = self._wants_refine()
-        if not self._wants_pipeline():
+        self.resident = self._wants_resident()
+        if self.resident is None and not self._wants_pipeline():
             return None
         if self.precond == "bj":
             if self.isolate is not None:
@@ -831,16 +876,19 @@ class SolveJob:
             self._redo_setup()
         check_every, _ = self._polls()
         budget = deferred_budget(self.expected_iterations, kind)
-        args = (self._pcgp_args if kind == "pcgp" else self._pcg2p_args)(ws, check_every, budget)
+        if self.resident is not None:
+            entry, args = "resident", self._resident_args(ws, budget)
+        else:
+            entry, args = kind, (self._pcgp_args if kind == "pcgp" else self._pcg2p_args)(ws, check_every, budget)
         s = stream_ptr()
-        _lib.call(f"efea_{kind}_start", *args, s)
-        return PendingSolve(self, ws, kind, args, s)
+        _lib.call(f"efea_{entry}_start", *args, s)
+        return PendingSolve(self, ws, kind, args, s, entry)
 
     def _run_bicgstab(self, ws: Workspace, raise_on_fail: bool) -> SolveInfo:
         """A non-symmetric system: right-preconditioned BiCGStab with the
         FP64 block-Jacobi inverse (``efea_solve_bicgstab``), to a relative
         residual of ``tol_residual``."""
-        self.precond, self.pipelined, self.refine = "bj", False, False
+        self.precond, self.pipelined, self.refine, self.resident = "bj", False, False, None
         self.setup(64)
         if self.before_solve is not None and self.before_solve():
             self.setup(64)
@@ -877,7 +925,7 @@ class SolveJob:
             cache[key] = CoarseSpace(self.A.pattern, cs0.target, nodes)
         self.x.copy_(self.x0)
         self.fallback = True
-        self.pipelined = False
+        self.pipelined, self.resident = False, None
         self.precision = 64
         self.refine = False
         self.precond = "two-level"
@@ -920,15 +968,16 @@ class PendingSolve:
     iterations, or a fallback solve), and work queued from it in between must
     be redone."""
 
-    def __init__(self, job: SolveJob, ws: Workspace, kind: str, args: tuple, stream: int):
+    def __init__(self, job: SolveJob, ws: Workspace, kind: str, args: tuple, stream: int, entry: str):
         self.job, self.ws, self.kind, self.args, self.stream = job, ws, kind, args, stream
+        self.entry = entry  # of the C functions: kind's pipelined solve, or "resident"
         self.resumed = False
 
     def finish(self, raise_on_fail: bool = True) -> SolveInfo:
         job = self.job
         raw = (C.c_double * 4)()
         resumed = C.c_int(0)
-        rc = _lib.call(f"efea_{self.kind}_finish", *self.args, self.stream, C.cast(raw, C.c_void_p),
+        rc = _lib.call(f"efea_{self.entry}_finish", *self.args, self.stream, C.cast(raw, C.c_void_p),
                        C.byref(resumed))
         si = job._conclude(self.ws, rc, job.info(raw), raise_on_fail)
         self.resumed = bool(resumed.value) or rc != 0

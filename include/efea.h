@@ -360,6 +360,93 @@ int efea_pcg2p_finish(int precision, int Nnode, int dof_n, int group, const int3
                       double tol_residual, double tol_anorm, int maxit, int check_every, int first_check,
                       void* stream, double* info, int* resumed);
 
+/* Resident PCG: the whole solve in one launch, FP64, for systems
+ * whose matrix fits the chip's registers (Chronopoulos and Gear's form of the
+ * preconditioned CG: the iterates and stopping test of efea_solve_pcg, and of
+ * efea_solve_pcg2 with a plan that has aggregates).  The plan belongs to the
+ * sparsity pattern (and its aggregates) and is built once.  A block of 512
+ * threads owns nloc = 512 / lanes * passes positions (lanes, slots and passes
+ * from efea_resident_shape); position p is node group p % (64 / lanes) of
+ * chunk p / (64 / lanes), and chunk c belongs to wave c % 8, pass c / 8.
+ *   rows (nblk * nloc): the node of each position, -1 for none;
+ *   lidx (nblk, passes, slots, 512): for thread t = 64 wave + lane of the node
+ *     and neighbour number (lane % lanes) + lanes * slot of its row, the
+ *     neighbour's position in the same block, or nloc + its place in the
+ *     block's halo list (0 where there is no such neighbour); with dof_n 1 the
+ *     node itself comes first (neighbour 0, then the others in row order) and
+ *     has no entry: slots - 1 of them, for slots 1, 2, ...;
+ *   self (nblk * nloc, dof_n 1): the node's place in its own row;
+ *   halo_ptr (nblk + 1), halo_ex: exchange numbers of each block's halo nodes;
+ *   pub (nblk * nloc): the exchange number of a position's node, -1 if no
+ *     other block reads it; nex exchange numbers in all, in position order:
+ *     block k's are pub_ptr[k] .. pub_ptr[k + 1] - 1 and belong to positions
+ *     pub_pos (within the block);
+ *   with aggregates (nagg > 0, else 0 and the pointers null), whose nodes
+ *     fill whole chunks in aggregate order: pieces are the runs of one
+ *     block's chunks of one aggregate, numbered through; piece_ptr (nblk + 1),
+ *     piece_agg (npiece), piece_chunk (2 npiece: first and past-last chunk of
+ *     its block), chunk_piece (nblk * 8 * passes: piece of each chunk within its block,
+ *     -1 for none); max_pieces: the most pieces of one block;
+ *   collect (ncollect * 256, with aggregates): what thread 256 + c of every
+ *     block reads of the restrictions the blocks publish per iteration, entries
+ *     collect[i * 256 + c], -1 for none (none after it either): offset |
+ *     destination << 16 | last << 31.  Block k publishes, at offset k * line,
+ *     three scalars and the restrictions of its pieces (nm values each; line =
+ *     3 + nm max_pieces rounded up to a multiple of 8).  A thread adds its
+ *     entries up to each one marked last and stores the sum at its destination:
+ *     component aggregate * nm + mode of the restriction from all pieces of the
+ *     aggregate, in block order.
+ * At most one block per CU (nblk <= the device's CU count and 256). */
+typedef struct efea_resident_plan {
+  int32_t dof_n, slots, passes;
+  int32_t nblk, max_halo, nex;
+  int32_t nagg, npiece, max_pieces, ncollect;
+  const int32_t* rows;
+  const uint16_t* lidx;
+  const int32_t* halo_ptr;
+  const int32_t* halo_ex;
+  const int32_t* pub;
+  const int32_t* pub_ptr;
+  const int32_t* pub_pos;
+  const int32_t* self;
+  const int32_t* piece_ptr;
+  const int32_t* piece_agg;
+  const int32_t* piece_chunk;
+  const int32_t* chunk_piece;
+  const int32_t* collect;
+} efea_resident_plan;
+/* The smallest kernel variant for rows of at most max_neighbours nodes (self
+ * included) with at least min_passes passes: returns 1 and its lanes per node,
+ * slots per lane and passes, or 0 when there is none. */
+int efea_resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, int* slots, int* passes);
+/* 1 if a block of the plan (sizes only; the pointers are not read) fits a CU's LDS. */
+int efea_resident_fits(const efea_resident_plan* plan);
+size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan);
+/* The solve; Minv FP64 (efea_bj_setup), rel / Ainv / ld as in efea_solve_pcg2
+ * (ignored without aggregates), info as in efea_solve_pcg.  A block waits at
+ * most wait_ms (<= 0: 250) for the others; a solve given up so, a refused
+ * launch and a breakdown return EFEA_ERR_NOCONV with status 2, and the caller
+ * redoes the solve from the same start with efea_solve_pcg[2].  The resident
+ * solves of a process follow one another on a device, also from several
+ * streams.  A call waits for the solve, not for what was queued behind it.
+ * efea_resident_start / efea_resident_finish are its deferred form, as
+ * efea_pcgp_start / efea_pcgp_finish: the start queues at most first_check
+ * iterations.  Replaces __Solver_1 (Simulations/Solvers.py:502-553) with
+ * _Solve_Axb's backends (Solvers.py:225-394), as efea_solve_pcg does. */
+int efea_solve_resident(const efea_resident_plan* plan, int Nnode, const int32_t* node_ptr, const double* values64,
+                        const uint8_t* known, const double* Minv, const double* rel, const double* Ainv, int ld,
+                        const double* b, double* x, void* workspace, size_t workspace_bytes, double tol_residual,
+                        double tol_anorm, int maxit, int first_check, double wait_ms, void* stream, double* info);
+int efea_resident_start(const efea_resident_plan* plan, int Nnode, const int32_t* node_ptr, const double* values64,
+                        const uint8_t* known, const double* Minv, const double* rel, const double* Ainv, int ld,
+                        const double* b, double* x, void* workspace, size_t workspace_bytes, double tol_residual,
+                        double tol_anorm, int maxit, int first_check, double wait_ms, void* stream);
+int efea_resident_finish(const efea_resident_plan* plan, int Nnode, const int32_t* node_ptr, const double* values64,
+                         const uint8_t* known, const double* Minv, const double* rel, const double* Ainv, int ld,
+                         const double* b, double* x, void* workspace, size_t workspace_bytes, double tol_residual,
+                         double tol_anorm, int maxit, int first_check, double wait_ms, void* stream, double* info,
+                         int* resumed);
+
 /* Timing harness of efea_solve_pcg2p's dominant kernel (the product pass:
  * n = A m, the eight vector updates, the dot-product and restriction
  * partials): reps launches back to back on `stream`, on the solve's chunks,

@@ -1,0 +1,190 @@
+"""Resident solves (``efea_solve_resident``, GPU tests): every kernel variant
+against the classic iteration on the same system, paused and continued solves
+against whole ones bit for bit, and the ways out (a block that waits too long,
+a zero right-hand side, NaN)."""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import easyfea_amd as ea
+from easyfea_amd import Models, Simulations, _lib
+from easyfea_amd import device as dv
+from easyfea_amd import resident as R
+from easyfea_amd.mesh import tetra4_box
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(mesh, dof_n, seed=0):
+    """(A, b, x0, known): an elastic stiffness, or a reaction-diffusion matrix."""
+    rng = np.random.default_rng(seed)
+    if dof_n > 1:
+        E = np.exp(rng.normal(0.0, 0.2, mesh.Ne))
+        simu = Simulations.Elastic(mesh, Models.Elastic.Isotropic(mesh.dim, E=E, v=0.3))
+        A = simu._device_K()
+    else:
+        simu = Simulations.Thermal(mesh, Models.Thermal(np.exp(rng.normal(0.0, 0.3, mesh.Ne)), 1.0))
+        K, M = simu._device_KC()
+        A = dv.DeviceCsr(K.pattern)
+        A.combine([(1.0, K), (float(mesh.Nn) ** (2 / mesh.dim) / 50, M)])
+    known = np.zeros(mesh.Nn * dof_n, dtype=np.uint8)
+    side = np.nonzero(mesh.coord[:, 0] == 0)[0]
+    known.reshape(-1, dof_n)[side] = 1
+    x0 = np.zeros(mesh.Nn * dof_n)
+    x0.reshape(-1, dof_n)[side] = rng.normal(size=(side.size, dof_n)) * 1e-3
+    return A, dv.to_dev(rng.normal(size=x0.size)), dv.to_dev(x0), dv.to_dev(known)
+
+
+def _run(A, b, x0, known, precond, pipelined):
+    job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond=precond, pipelined=pipelined)
+    return job, job.run(raise_on_fail=False)
+
+
+def _close(x, y, known):
+    assert torch.equal(x[known != 0], y[known != 0])
+    return float(torch.linalg.vector_norm(x - y) / torch.linalg.vector_norm(y))
+
+
+Q, T, H = ea.quad4_rectangle, ea.tri3_rectangle, ea.hexa8_box
+CASES = [  # mesh, dof_n, preconditioner, (slots, passes)
+    (lambda: Q(1, 1, 1, 1), 2, "bj", (4, 1)),
+    (lambda: Q(4, 1, 60, 3), 2, "bj", (5, 1)),           # one block
+    (lambda: Q(1, 1, 15, 15), 2, "bj", (5, 1)),          # 256 nodes: one full block
+    (lambda: Q(1, 1, 32, 31), 2, "two-level", (5, 1)),
+    (lambda: T(1, 1, 33, 47), 2, "two-level", (4, 1)),
+    (lambda: T(1, 1, 290, 250), 2, "two-level", (4, 2)),
+    (lambda: Q(1, 1, 290, 250), 2, "two-level", (5, 2)),
+    (lambda: T(1, 1, 400, 420), 2, "bj", (4, 4)),
+    (lambda: Q(1, 1, 400, 420), 2, "two-level", (5, 4)),
+    (lambda: T(1, 1, 40, 30), 1, "bj", (7, 1)),
+    (lambda: T(1, 1, 420, 400), 1, "bj", (7, 2)),
+    (lambda: T(1, 1, 600, 600), 1, "bj", (7, 4)),
+    (lambda: Q(1, 1, 350, 353), 1, "bj", (9, 1)),
+    (lambda: Q(1, 1, 420, 400), 1, "bj", (9, 2)),
+    (lambda: Q(1, 1, 700, 610), 1, "bj", (9, 4)),
+    (lambda: Q(1, 1, 730, 720), 1, "bj", (9, 9)),
+    (lambda: T(1, 1, 730, 720), 1, "bj", (7, 9)),
+    (lambda: H(1, 1, 1, 7, 9, 8), 1, "bj", (28, 1)),
+    (lambda: H(1, 1, 1, 55, 54, 53), 1, "bj", (28, 2)),
+    (lambda: tetra4_box(1, 1, 1, 9, 9, 9), 1, "bj", (16, 1)),
+    (lambda: tetra4_box(1, 1, 1, 54, 55, 53), 1, "bj", (16, 2)),
+    (lambda: H(1, 1, 1, 5, 6, 4), 3, "bj", (7, 1)),
+    (lambda: H(1, 1, 1, 20, 19, 21), 3, "two-level", (7, 1)),
+    (lambda: H(1, 1, 1, 30, 31, 29), 3, "two-level", (7, 1)),
+    (lambda: tetra4_box(1, 1, 1, 17, 18, 17), 3, "two-level", (4, 1)),
+    (lambda: tetra4_box(1, 1, 1, 35, 34, 33), 3, "two-level", (4, 2)),
+    (lambda: tetra4_box(1, 1, 1, 6, 5, 4), 3, "bj", (4, 1)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_resident_matches_classic(case):
+    make, dof_n, precond, variant = CASES[case]
+    A, b, x0, known = _system(make(), dof_n)
+    job, info = _run(A, b, x0, known, precond, "auto")
+    p = job.resident.plan
+    print(f"{A.Nn} nodes: {p.nblk} blocks, {info.iterations} iterations", flush=True)
+    assert (p.slots, p.passes) == variant
+    assert info.status == 1 and info.resident and not info.fallback
+    classic, ci = _run(A, b, x0, known, precond, False)
+    assert not ci.resident and abs(info.iterations - ci.iterations) <= 2 + ci.iterations // 50
+    # both stop at an estimated 1e-10 in the energy norm
+    assert _close(job.x, classic.x, known) < 1e-8
+    assert info.rel_residual < 10 * max(ci.rel_residual, 1e-12)
+    again, ai = _run(A, b, x0, known, precond, "auto")
+    assert torch.equal(again.x, job.x) and ai.iterations == info.iterations
+
+
+@pytest.mark.parametrize("case", [2, 3, 6, 13, 15, 23, 26])
+def test_paused_solve_continues_bit_for_bit(case):
+    make, dof_n, precond, _ = CASES[case]
+    A, b, x0, known = _system(make(), dof_n)
+    whole, wi = _run(A, b, x0, known, precond, "auto")
+    for expected in (1, 9, wi.iterations - 4, wi.iterations):
+        job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond=precond,
+                          expected_iterations=max(1, expected))
+        pending = job.start()
+        assert pending is not None and pending.entry == "resident"
+        info = pending.finish()
+        queued = dv.deferred_budget(max(1, expected), pending.kind)
+        assert pending.resumed == (queued <= wi.iterations)  # the test that ends it follows the last one
+        assert torch.equal(job.x, whole.x)
+        assert (info.iterations, info.rel_residual, info.status) == (wi.iterations, wi.rel_residual, 1)
+
+
+def test_a_block_that_waits_too_long_gives_up(monkeypatch):
+    """A wait limit no exchange can meet: the solve fails, every wait ends, and
+    the classic iteration redoes it from the same start."""
+    A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
+    _, ci = _run(A, b, x0, known, "two-level", False)
+    monkeypatch.setattr(dv, "RESIDENT_WAIT_MS", 1e-9)
+    job, info = _run(A, b, x0, known, "two-level", "auto")
+    assert info.status == 1 and info.fallback and not info.resident and info.iterations == ci.iterations
+    assert job.pipeline_failure[0] == _lib.ERR_NOCONV and "waited" in job.pipeline_failure[1]
+    monkeypatch.undo()
+    _, info = _run(A, b, x0, known, "two-level", "auto")
+    assert info.status == 1 and info.resident
+
+
+@pytest.mark.parametrize("dof_n,precond", [(1, "bj"), (2, "two-level")])
+def test_zero_and_non_finite_right_hand_sides(dof_n, precond):
+    A, b, x0, known = _system(Q(1, 1, 40, 40), dof_n)
+    zero = torch.zeros_like(b)
+    job, info = _run(A, zero, torch.zeros_like(b), known, precond, "auto")
+    assert info.status == 1 and info.iterations == 0 and not job.x.any()
+    b[17 * dof_n] = float("nan")
+    for pipelined in ("auto", False):
+        _, info = _run(A, b, x0, known, precond, pipelined)
+        assert info.status == 2
+
+
+def test_two_threads_on_their_own_streams():
+    """Solves of two threads at once take the chip in turn, with the results of
+    one after the other."""
+    import threading
+
+    systems = [_system(Q(1, 1, 90 + 7 * k, 80), 2, seed=k) for k in range(2)]
+    want = [_run(*s, "two-level", "auto")[0].x for s in systems]
+    got, errors = [[], []], []
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(6):
+                    job, info = _run(*systems[k], "two-level", "auto")
+                    got[k].append((info.resident, job.x))
+        except Exception as exc:  # shown by the assertion below
+            errors.append(exc)
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for k in range(2):
+        for resident, x in got[k]:
+            assert resident and torch.equal(x, want[k])
+
+
+def test_refused_arguments():
+    lib = _lib.load()
+    fake, info = 0x1000, (C.c_double * 4)()
+    plan = _lib.ResidentPlan(dof_n=2, slots=5, passes=1, nblk=4, max_halo=10, nex=10, rows=fake, lidx=fake,
+                             halo_ptr=fake, halo_ex=fake, pub=fake, pub_ptr=fake, pub_pos=fake, self=fake)
+    args = [100, fake, fake, None, fake, None, None, 0, fake, fake, fake, 1 << 30, 1e-12, 1e-9, 10, 0, 0.0, None]
+    assert lib.efea_solve_resident(C.byref(plan), 0, *args[1:], info) == -1
+    plan.slots = 6
+    assert lib.efea_solve_resident(C.byref(plan), *args, info) == -1 and "no kernel" in _lib.last_error()
+    plan.slots, plan.nblk = 5, 300
+    assert lib.efea_solve_resident(C.byref(plan), *args, info) == -1
+    plan.nblk, plan.max_halo = 4, 20000  # more LDS than a CU has
+    assert lib.efea_resident_fits(C.byref(plan)) == 0
+    plan.max_halo, args[11] = 10, 16
+    assert lib.efea_solve_resident(C.byref(plan), *args, info) == -4
+    assert R.shape(2, 9, 1) == (2, 5, 1)
