@@ -725,24 +725,40 @@ class Elastic(_Simu):
             self._M = None
 
     def Assembly(self):
-        """Element stiffness on the device and deterministic scatter."""
+        """The stiffness on the device, summed per entry in increasing element
+        order: straight into the CSR values, or (where
+        ``DeviceMesh.row_incidence`` has no plan) through element matrices and
+        the deterministic scatter."""
         dev = self.dev
         A = dev.csr_map(self.model.dim)
-        Ke = A.new_entries()
         tab, nPg = dev.tables(MatrixType.rigi)
-        if isinstance(self.model, Anisotropic):
-            # a general constitutive matrix: B^T C B on the matrix cores
+        m = self.model
+        general = isinstance(m, Anisotropic)
+        if general:
             if dev.code not in (_lib.ELEM_CODE["HEXA8"], _lib.ELEM_CODE["TETRA10"]):
                 raise NotImplementedError("anisotropic laws: HEXA8 and TETRA10 meshes on the device")
-            C = to_dev(np.ascontiguousarray(self.model.C).reshape(-1))
-            _lib.call("efea_elastic_ke_dense", dev.code, dev.Ne, ptr(dev.connect), ptr(dev.coord), ptr(tab), nPg,
-                      ptr(C), 1 if self.model.isHeterogeneous else 0, None, 0, 0.0, ptr(Ke), stream_ptr())
+            C = to_dev(np.ascontiguousarray(m.C).reshape(-1))
         else:
-            E = to_dev(self.model._E_array())
-            _lib.call("efea_elastic_ke", dev.code, 64, dev.Ne, ptr(dev.connect), ptr(dev.coord), ptr(tab), nPg,
-                      ptr(E), 1 if self.model.isHeterogeneous else 0, self.model.v, int(self.model.planeStress),
-                      self.model.thickness, ptr(Ke), stream_ptr())
-        A.scatter(Ke)
+            E = to_dev(m._E_array())
+        het = 1 if m.isHeterogeneous else 0
+        rows = dev.row_incidence(m.dim)
+        if rows is not None:
+            inc_ptr, inc, pos = rows
+            law = (None, 0, 0.0, 0, 1.0, ptr(C), het) if general else \
+                (ptr(E), het, m.v, int(m.planeStress), m.thickness, None, 0)
+            _lib.call("efea_elastic_assemble", dev.code, dev.Nn, ptr(A.node_ptr), A.host.max_neighbours, ptr(inc_ptr),
+                      ptr(inc), ptr(pos), ptr(dev.connect), ptr(dev.coord), ptr(tab), nPg, *law, ptr(A.values),
+                      stream_ptr())
+            A.changed()
+        else:
+            Ke = A.new_entries()
+            if general:  # B^T C B on the matrix cores
+                _lib.call("efea_elastic_ke_dense", dev.code, dev.Ne, ptr(dev.connect), ptr(dev.coord), ptr(tab), nPg,
+                          ptr(C), het, None, 0, 0.0, ptr(Ke), stream_ptr())
+            else:
+                _lib.call("efea_elastic_ke", dev.code, 64, dev.Ne, ptr(dev.connect), ptr(dev.coord), ptr(tab), nPg,
+                          ptr(E), het, m.v, int(m.planeStress), m.thickness, ptr(Ke), stream_ptr())
+            A.scatter(Ke)
         self._K = A
         self._needUpdate = False
         return A

@@ -114,6 +114,10 @@ int pp_iter_bench(int, int, int, int, const int*, const int*, const double*, con
                   const unsigned char*, int, const double*, int, const int*, const int*, int, double*, void*, int,
                   hipStream_t);
 
+int assemble_max_neighbours(int);
+int elastic_assemble(int, int, const int*, int, const int*, const int*, const unsigned short*, const int*,
+                     const double*, const double*, int, const double*, int, double, int, double, const double*, int,
+                     double*, hipStream_t);
 int elastic_ke_dense(int, int64_t, const int*, const double*, const double*, int, const double*, int, const double*,
                      int, double, double*, hipStream_t);
 }  // namespace efea
@@ -186,6 +190,21 @@ int efea_elastic_ke_dense(int elem_type, int64_t Ne, const int32_t* connect, con
   }
   return elastic_ke_dense(elem_type, Ne, connect, coord, tables, nPg, D, D_stride, E, E_stride, nu, Ke,
                           STREAM(stream));
+}
+
+int efea_assemble_max_neighbours(int elem_type) { return assemble_max_neighbours(elem_type); }
+
+int efea_elastic_assemble(int elem_type, int Nn, const int32_t* node_ptr, int max_neighbours, const int32_t* inc_ptr,
+                          const int32_t* inc, const uint16_t* pos, const int32_t* connect, const double* coord,
+                          const double* tables, int nPg, const double* E, int E_stride, double nu, int plane_stress,
+                          double thickness, const double* D, int D_stride, double* values, void* stream) {
+  if (Nn <= 0 || max_neighbours <= 0 || !node_ptr || !inc_ptr || !inc || !pos || !connect || !coord || !tables ||
+      !values || (!E && !D)) {
+    set_error("efea_elastic_assemble: null pointer or empty mesh");
+    return EFEA_ERR_ARG;
+  }
+  return elastic_assemble(elem_type, Nn, node_ptr, max_neighbours, inc_ptr, inc, pos, connect, coord, tables, nPg, E,
+                          E_stride, nu, plane_stress, thickness, D, D_stride, values, STREAM(stream));
 }
 
 int efea_elastic_strain_stress(int elem_type, int64_t Ne, const int32_t* connect, const double* coord,

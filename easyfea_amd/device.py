@@ -139,6 +139,22 @@ class DeviceMesh:
             c = self._shared.__dict__["incidence"] = (to_dev(ptr_), to_dev(cols[order].astype(np.int32)))
         return c
 
+    def row_incidence(self, dof_n: int) -> Optional[tuple]:
+        """(inc_ptr, inc, pos) of ``efea_elastic_assemble`` on the device: per
+        node its elements in increasing order (``element * 16 + the node's
+        number in it``) and, per incidence, the places of the element's nodes
+        in the node's row.  Mesh data, built once.  None where the assembly by
+        rows does not apply: rows longer than a block's LDS holds, an element
+        that names a node twice (two lanes would add to one slot), more
+        elements than the code's 27 bits."""
+        d = self._shared.__dict__
+        if "row_incidence" not in d:
+            p = self.pattern(dof_n)
+            fits = p.host.max_neighbours <= _lib.load().efea_assemble_max_neighbours(self.code) and self.Ne < 1 << 27
+            d["row_incidence"] = row_incidence(self.connect, self.Nn, p.node_ptr, p.node_cols) if fits else None
+            torch.cuda.current_stream().synchronize()  # as an upload: any stream may use it from here on
+        return d["row_incidence"]
+
     def node_values(self, values_e: torch.Tensor) -> torch.Tensor:
         """Element values (Ne, k) -> node values (Nn, k) (``Mesh.Get_Node_Values``)."""
         v = values_e.reshape(self.Ne, -1).contiguous()
@@ -172,6 +188,22 @@ class DeviceMesh:
         if dof_n not in v:
             v[dof_n] = DeviceVecMap(build_vec_map(self.connect_np, self.Nn, dof_n))
         return v[dof_n]
+
+
+def row_incidence(connect: torch.Tensor, Nn: int, node_ptr: torch.Tensor, node_cols: torch.Tensor) -> Optional[tuple]:
+    """See ``DeviceMesh.row_incidence`` (torch, on the inputs' device)."""
+    nPe = connect.shape[1]
+    con = connect.long()
+    node, order = torch.sort(con.reshape(-1), stable=True)  # by node, elements increasing
+    e = order // nPe
+    if bool(((node[1:] == node[:-1]) & (e[1:] == e[:-1])).any()):
+        return None
+    nodes = torch.arange(Nn + 1, device=con.device)
+    inc_ptr = torch.searchsorted(node, nodes, out_int32=True)
+    start = node_ptr.long()
+    keys = torch.repeat_interleave(nodes[:-1] * Nn, start[1:] - start[:-1], output_size=len(node_cols)) + node_cols
+    pos = torch.searchsorted(keys, node[:, None] * Nn + con[e]) - start[node][:, None]
+    return inc_ptr, (e * 16 + order % nPe).int(), pos.to(torch.int16)
 
 
 class DeviceVecMap:
@@ -369,6 +401,10 @@ class DeviceCsr:
         assert Ke.numel() == self.n_entries and Ke.dtype == torch.float64
         _lib.call("efea_csr_scatter", 64, self.nnz, ptr(self.seg), ptr(self.perm), ptr(Ke), ptr(self.values),
                   stream_ptr())
+        self.changed()
+
+    def changed(self) -> None:
+        """The values were rewritten: drops what was formed from the old ones."""
         self.values32 = None
         self.corr32 = None
         self.version += 1
@@ -382,9 +418,7 @@ class DeviceCsr:
             c, X = terms[k] if k < len(terms) else (0.0, None)
             args += [float(c), ptr(X.values) if X is not None else None]
         _lib.call("efea_lincomb", self.nnz, *args, ptr(self.values), stream_ptr())
-        self.values32 = None
-        self.corr32 = None
-        self.version += 1
+        self.changed()
 
     def make_fp32(self) -> torch.Tensor:
         """FP32 copy of the values and its row-sum correction (``efea_split_f32``)."""

@@ -61,6 +61,24 @@ int efea_elastic_ke_dense(int elem_type, int64_t Ne, const int32_t* connect, con
                           const double* tables, int nPg, const double* D, int D_stride, const double* E, int E_stride,
                           double nu, double* Ke, void* stream);
 
+/* The global elastic stiffness straight into the CSR value array (no element
+ * matrices): values of the canonical CSR of Nn nodes (node_ptr: node
+ * adjacency offsets, rows of at most max_neighbours nodes), summed per entry in
+ * increasing element order.  Per node, inc_ptr / inc list its elements
+ * (increasing) as element * 16 + the node's number in it, and pos (nPe per
+ * incidence) the place of each of the element's nodes in the node's row.
+ * Isotropic with E (E_stride 0 / 1) and nu (plane_stress, thickness in 2D) as
+ * efea_elastic_ke, or with D (Kelvin-Mandel 6 x 6, D_stride 0 / 1; 3D) as
+ * efea_elastic_ke_dense.  EFEA_ERR_SIZE when a block's rows do not fit its LDS
+ * (max_neighbours above efea_assemble_max_neighbours).  Replaces
+ * Operators.Bilinear.LinearizedElasticity (FEM/Operators/Bilinear.py:62-79)
+ * followed by _Simu.__Assemble_csr (Simulations/_simu.py:1051-1055). */
+int efea_elastic_assemble(int elem_type, int Nn, const int32_t* node_ptr, int max_neighbours, const int32_t* inc_ptr,
+                          const int32_t* inc, const uint16_t* pos, const int32_t* connect, const double* coord,
+                          const double* tables, int nPg, const double* E, int E_stride, double nu, int plane_stress,
+                          double thickness, const double* D, int D_stride, double* values, void* stream);
+int efea_assemble_max_neighbours(int elem_type);
+
 /* Linear-elastic post-processing per element (Simulations/_elastic.py:229-380,
  * Models/Elastic/_laws.py:127-185, Models/_utils.py:302-434): at each stiffness
  * integration point eps = B u_e (Kelvin-Mandel) and sig = C eps (isotropic,
