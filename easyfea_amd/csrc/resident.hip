@@ -56,8 +56,8 @@
 // and barriers.  Measured per iteration, the launch-per-step solve before and
 // this one: QUAD4 32^2 (8 blocks) 15.9 -> 4.8 us, 360 x 39 (64) 16.5 -> 5.6,
 // TRI3 251 x 249 (256) 22 -> 6.8, notched TRI3 200^2 (161) 20 -> 7.6, HEXA8
-// 30^3 (236) 42.6 -> 12.6, scalar QUAD4 700^2 (240) 28 -> 7.6; block Jacobi on
-// 360 x 39 10.2 -> 4.0.
+// 30^3 (236) 42.6 -> 12.6, scalar QUAD4 700^2 (240) 28 -> 7.6, 1024^2 (229)
+// 50 -> 16; block Jacobi on 360 x 39 10.2 -> 4.0.
 //
 // It replaces the same call as efea_solve_pcg: __Solver_1
 // (Simulations/Solvers.py:502-553) with _Solve_Axb's backends
@@ -252,7 +252,7 @@ __host__ __device__ inline ResLds res_lds(const ResidentPlan& P, int S, int NP, 
   o += o & 1;
   L.rows = o; o += (TWO && cache_rows) ? P.max_pieces * NM * nc : 0;
   L.item = o; o += TWO ? P.ncollect * CT / 2 : 0;
-  L.idx = o; o += BIG ? NP * (S - 1) * RT / 4 : 0;
+  L.idx = o; o += BIG ? NP * ((S + 2) / 4) * RT : 0;
   L.p = o; o += BIG ? nloc : 0;
   L.total = o;
   return L;
@@ -262,6 +262,7 @@ struct ResWork {
   double *r, *u, *p, *s;   // a paused solve's vectors
   double *z, *zs;          // its rows of Ac^-1 P^T r and of the same for s
   double* xp;              // BIG: x in position order
+  double* vs;              // BIG: the values of the streamed passes, per block, pass and slot
   u64 *hx, *pay;
   PcgState* st;
 };
@@ -289,14 +290,26 @@ __global__ void __launch_bounds__(256) k_res_empty(int64_t n, u64* __restrict__ 
   if (blockIdx.x == 0 && threadIdx.x == 0) out->failed = 0;
 }
 
-// BIG (scalar, most passes): the values take two thirds of the registers, so
-// the neighbour positions and p live in LDS, x in L2 (updated while the halo
-// is on its way), u only in LDS, and B^-1 is the division by the diagonal.
+// BIG (scalar, most passes): the block's neighbour positions and p live in
+// LDS, x in L2 (updated while the halo is on its way), u only in LDS, and B^-1
+// is the division by the diagonal.  Of the values at most 72 registers' worth
+// stay (9 slots: 4 passes of 9), the other passes are read from the cache in
+// every product, laid out for it at the start: with more kept the compiler
+// spilled, and a spilled word waits behind the streamed ones.  QUAD4 1024^2
+// scalar, 164 iterations: 4 passes kept 10.9 ms for three solves, 6 kept 11.2,
+// 7 kept 12.6, all 9 kept (180 words per thread spilled) 25.4; launch-per-step
+// 27.7.  It is bound by the product: 13,000 of 33,000 cycles per iteration,
+// LDS reads and the latency of the streamed passes.
+template <int S, int NP, bool BIG>
+struct ResPasses {
+  static constexpr int KEPT = !BIG || 2 * S * NP <= 72 ? NP : 72 / (2 * S);
+};
 template <int DN, int S, int NP, bool TWO, bool BIG>
 __global__ void __launch_bounds__(RT, 2)
 k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   constexpr int NM = Modes<DN>::NM, G = ResLanes<DN>::G, NPC = 64 / G, NLOC = RT / G * NP;
   constexpr int SN = ResSlots<DN, S>::N, S2 = (SN + 1) / 2, NR = BIG ? 1 : NP;
+  constexpr int NV = ResPasses<S, NP, BIG>::KEPT;  // passes whose values stay in registers
   static_assert(!BIG || (DN == 1 && !TWO), "BIG is scalar block Jacobi");
   extern __shared__ double lds[];
   __shared__ double ring[RING], lsc[16];  // lsc: sums of the scalars, 4 per collecting wave
@@ -309,7 +322,9 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   double* lz = lds + L.z;
   double* lzs = lds + L.zs;
   double* lrow = lds + L.rows;
-  unsigned short* lidx = (unsigned short*)(lds + L.idx);
+  // BIG: the neighbours' byte offsets in lu, four to a word
+  constexpr int SH = (SN + 3) / 4;
+  u64* lidx = (u64*)(lds + L.idx);
   double* lp = lds + L.p;
 
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, q = lane / G, g = lane % G;
@@ -319,12 +334,25 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   const bool own = g < DN;
   if (t == 0) lfail = 0;
   if (t < RING) ring[t] = 0;
-  auto at = [&](int p) { return (p * RNW + wv) * NPC + q; };  // the lane's position of pass p
+  // the lane's position of pass p
+  auto at = [&](int p) { return G == 1 ? p * RT + t : (p * RNW + wv) * NPC + q; };
+  // a uniform address, formed anew each time: the loop's own copies of what is
+  // added to it would fill the registers
+  // between passes: several passes' loads in flight would spill
+  auto fence = [] {
+    if constexpr (NP > 1) __builtin_amdgcn_sched_barrier(0);
+  };
+  using Global = __attribute__((address_space(1))) double;
+  auto fresh = [](double* a) {
+    auto* f = (Global*)a;
+    asm volatile("" : "+s"(f));
+    return f;
+  };
 
   // ---- the block's nodes, matrix values and neighbour positions
   int node[NR], pubx[NR], piece[NR];
   unsigned li[NR][BIG ? 1 : S2];
-  double v[NP][S][DN][DN], Mi[NR][DN];
+  double v[NV][S][DN][DN], Mi[NR][DN], dg[NP - NV + 1];
   double xv[NR], rv[NP], pv[NR], sv[NP], uv[NR];
   unsigned kmask = 0;
 #pragma unroll
@@ -336,6 +364,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     const int p0 = A.node_ptr[n], cnt = A.node_ptr[n + 1] - p0;
     const int64_t base = (int64_t)DN * DN * p0;
     const int self = DN == 1 ? P.self[gp] : 0;
+    double* vs = W.vs + ((int64_t)blk * (NP - NV) + (p - NV)) * S * RT + t;  // a streamed pass
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       int j = g + s * G;
@@ -347,20 +376,31 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
 #pragma unroll
         for (int b = 0; b < DN; ++b) {
           const double vv = A.vals[base + (int64_t)a * DN * cnt + (int64_t)jj * DN + b];
-          v[p][s][a][b] = ok ? vv : 0.0;
+          if (p < NV) {
+            v[p][s][a][b] = ok ? vv : 0.0;
+          } else {
+            vs[s * RT] = ok ? vv : 0.0;
+            if (s == 0) dg[p - NV] = ok ? vv : 0.0;
+          }
         }
     }
     if constexpr (!BIG) {
 #pragma unroll
       for (int s = 0; s < S2; ++s) li[p][s] = 0;
     }
+    u64 four = 0;
 #pragma unroll
     for (int s = 0; s < SN; ++s) {
       const unsigned i = P.lidx[(((int64_t)blk * NP + p) * SN + s) * RT + t];
-      if constexpr (BIG)
-        lidx[(p * SN + s) * RT + t] = (unsigned short)i;
-      else
+      if constexpr (BIG) {
+        four |= (u64)(8 * i) << (16 * (s & 3));
+        if ((s & 3) == 3 || s == SN - 1) {
+          lidx[(p * SH + s / 4) * RT + t] = four;
+          four = 0;
+        }
+      } else {
         li[p][s / 2] |= i << (16 * (s & 1));
+      }
     }
     const int64_t i = (int64_t)n * DN + (own ? g : 0);
     const bool act = have && own;
@@ -384,7 +424,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
         for (int d = 0; d < 3; ++d) lrel[at(p) * 3 + d] = have ? A.rel[3 * (int64_t)n + d] : 0.0;
       }
     }
-    if constexpr (NP > 1) __builtin_amdgcn_sched_barrier(0);
+    fence();
   }
   const int pc0 = TWO ? P.piece_ptr[blk] : 0, npc = TWO ? P.piece_ptr[blk + 1] - pc0 : 0;
   const int nrow = npc * NM, mine = 3 + nrow;  // rows of Ac^-1, published sums
@@ -422,13 +462,9 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
 
   // the position in lu of slot s of pass p (after the first, own, slot of a scalar row)
   auto nb = [&](int p, int s) -> int {
-    if constexpr (BIG) {
-      return lidx[(p * SN + s) * RT + t];
-    } else {
-      unsigned w = li[p][s / 2];
-      asm volatile("" : "+v"(w));  // unpacked here each time: unpacked once, they would fill the registers
-      return (int)((w >> (16 * (s & 1))) & 0xffffu);
-    }
+    unsigned w = li[p][s / 2];
+    asm volatile("" : "+v"(w));  // unpacked here each time: unpacked once, they would fill the registers
+    return (int)((w >> (16 * (s & 1))) & 0xffffu);
   };
   // the own values of lu to the other blocks (halo buffer k & 1; the other one
   // and the sums after next are emptied)
@@ -480,8 +516,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   };
   // component g of A lu at the lane's node (owner lanes), 0 at known rows
   auto product = [&](double (&y)[NP]) {
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
+    auto pass = [&](int p, const double (&vp)[S][DN][DN]) {
       double sum[DN];
 #pragma unroll
       for (int a = 0; a < DN; ++a) sum[a] = 0;
@@ -494,7 +529,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
 #pragma unroll
         for (int a = 0; a < DN; ++a)
 #pragma unroll
-          for (int b = 0; b < DN; ++b) sum[a] += v[p][s][a][b] * ub[b];
+          for (int b = 0; b < DN; ++b) sum[a] += vp[s][a][b] * ub[b];
       }
       double r;
       if constexpr (DN == 1) {
@@ -511,8 +546,53 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
         r = g == 0 ? sum[0] : (g == 1 ? sum[1] : sum[2]);
       }
       y[p] = ((kmask >> p) & 1u) ? 0.0 : r;
-      // one pass's LDS reads in flight at a time: several passes' would spill
-      if constexpr (NP > 1) __builtin_amdgcn_sched_barrier(0);
+      // formed here: sunk to its first use, past a branch, it would keep every operand live
+      asm volatile("" : "+v"(y[p]));
+      fence();
+    };
+    if constexpr (!BIG) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) pass(p, v[p]);
+    } else {
+      // a streamed pass's values are on their way while the passes before it are
+      // formed, a pass's offsets while the one before is
+      constexpr int NS = NP - NV, ND = NS > 0 ? NS : 1;
+      u64 ix[SH];
+      auto split = [](int i) { return (i * NV + ND - 1) / ND; };  // kept passes before streamed pass i
+      auto offsets = [&](int p, u64 (&w)[SH]) {
+#pragma unroll
+        for (int h = 0; h < SH; ++h) w[h] = lidx[(p * SH + h) * RT + t];
+      };
+      auto big = [&](int p, int next, const double (&vp)[S][DN][DN]) {
+        double ub[S];
+        ub[0] = lu[at(p)];
+#pragma unroll
+        for (int s = 1; s < S; ++s)
+          ub[s] = *(const double*)((const char*)lu + (unsigned)((ix[(s - 1) / 4] >> (16 * ((s - 1) & 3))) & 0xffffu));
+        offsets(next, ix);
+        fence();
+        double sum = 0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) sum += vp[s][0][0] * ub[s];
+        y[p] = ((kmask >> p) & 1u) ? 0.0 : sum;
+        asm volatile("" : "+v"(y[p]));  // as above
+        fence();
+      };
+      offsets(0, ix);
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        double w[S][DN][DN];
+        if constexpr (NS > 0) {
+          const Global* vs = fresh(W.vs + (int64_t)blk * NS * S * RT);
+#pragma unroll
+          for (int s = 0; s < S; ++s) w[s][0][0] = vs[(unsigned)((i * S + s) * RT + t)];
+          fence();
+        }
+        const int p0 = split(i), p1 = split(i + 1);
+#pragma unroll
+        for (int p = p0; p < p1; ++p) big(p, NS > 0 && p + 1 == p1 ? NV + i : (p + 1 < NP ? p + 1 : 0), v[p]);
+        if constexpr (NS > 0) big(NV + i, i + 1 < NS ? (p1 < split(i + 2) ? p1 : NV + i + 1) : 0, w);
+      }
     }
   };
   // block sums of three scalars and of P^T rest per piece, published as sums k,
@@ -520,7 +600,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   auto sums = [&](double s0, double s1, double s2, const double (&rest)[NP], int k, bool read) -> bool {
     // the values' place in wave_sum4's rows
     const int row = lane >> 4, w4 = row == 1 ? 2 : (row == 2 ? 1 : row);
-    constexpr int CS = RNW * NP;  // column of lch: a value of each chunk
+    constexpr int CS = TWO ? RNW * NP : RNW;  // column of lch: a value of each chunk
     if constexpr (TWO) {
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
@@ -650,7 +730,10 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     if constexpr (TWO) __syncthreads();
     if constexpr (BIG) {
 #pragma unroll
-      for (int p = 0; p < NP; ++p) lu[at(p)] = ((kmask >> p) & 1u) ? 0.0 : rv[p] / v[p][0][0][0];
+      for (int p = 0; p < NP; ++p) {
+        lu[at(p)] = ((kmask >> p) & 1u) ? 0.0 : rv[p] / (p < NV ? v[p < NV ? p : 0][0][0][0] : dg[p < NV ? 0 : p - NV]);
+        fence();
+      }
     } else {
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
@@ -686,12 +769,12 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   // BIG: x += a_prev p of the last step
   auto update_x = [&]() {
     if constexpr (BIG) {
-      double* xp = W.xp + (int64_t)blk * NLOC;
+      Global* xp = fresh(W.xp + (int64_t)blk * NLOC);
       double xo[NP];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) xo[p] = xp[at(p)];
+      for (int p = 0; p < NP; ++p) xo[p] = xp[(unsigned)at(p)];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) xp[at(p)] = xo[p] + a_prev * lp[at(p)];
+      for (int p = 0; p < NP; ++p) xp[(unsigned)at(p)] = xo[p] + a_prev * lp[at(p)];
       xpend = false;
     }
   };
@@ -732,6 +815,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
           pv[p] = W.p[i];
         }
       }
+      fence();
     }
     __syncthreads();
   } else {
@@ -742,6 +826,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
       for (int p = 0; p < NP; ++p) {
         const int nd = P.rows[(int64_t)blk * NLOC + at(p)];
         xp[at(p)] = nd >= 0 ? A.x[nd] : 0.0;
+        fence();
       }
       x_to_lu();
     }
@@ -756,6 +841,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
         if (!((kmask >> p) & 1u)) rv[p] = A.b[(int64_t)nd * DN + g] - y[p];
         ax += (BIG ? lu[at(p)] : xv[BIG ? 0 : p]) * y[p];
         r2 += rv[p] * rv[p];
+        fence();
       }
       good = sums(ax, r2, 0.0, rv, k, true);
     }
@@ -829,6 +915,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
       rv[p] -= alpha * sv[p];
       if constexpr (BIG) {
         lp[at(p)] = lu[at(p)] + beta * lp[at(p)];
+        fence();
       } else {
         pv[p] = uv[p] + beta * pv[p];
         xv[p] += alpha * pv[p];
@@ -856,6 +943,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
           W.s[i] = sv[p];
         }
       }
+      fence();
     }
     if constexpr (TWO) {
       if (!done) {
@@ -877,6 +965,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
       const int nd = BIG ? P.rows[(int64_t)blk * NLOC + at(p)] : node[BIG ? 0 : p];
       const double r = ((kmask >> p) & 1u) ? 0.0 : A.b[(int64_t)nd * DN + g] - y[p];
       r2 += r * r;
+      fence();
     }
     good = sums(r2, 0.0, 0.0, y, k, blk == 0);
   }
@@ -915,11 +1004,32 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   }
 }
 
+// The kernel variants: dof_n, slots per lane, passes, BIG.  A
+// block holds RT / lanes * passes nodes, of at most lanes * slots neighbours
+// each; the largest pass count of each slot count is what 256 registers hold.
+#define EFEA_RESIDENT(X)                                                                    \
+  X(1, 7, 1, false) X(1, 7, 2, false) X(1, 7, 4, false) X(1, 7, 9, true)                     \
+  X(1, 9, 1, false) X(1, 9, 2, false) X(1, 9, 4, false) X(1, 9, 9, true)                     \
+  X(1, 16, 1, false) X(1, 16, 2, false) X(1, 28, 1, false) X(1, 28, 2, false)               \
+  X(2, 4, 1, false) X(2, 4, 2, false) X(2, 4, 4, false)                                     \
+  X(2, 5, 1, false) X(2, 5, 2, false) X(2, 5, 4, false) X(2, 8, 1, false) X(2, 8, 2, false) \
+  X(3, 4, 1, false) X(3, 4, 2, false) X(3, 7, 1, false)
+
 static inline int res_modes(int dof_n) { return dof_n == 1 ? 1 : (dof_n == 2 ? 3 : 6); }
 
 // BIG's x in position order (allotted for every scalar plan).
 static inline size_t res_xp_bytes(const ResidentPlan& P) {
   return P.dof_n == 1 ? align256(8 * (size_t)P.nblk * RT * P.passes) : 0;
+}
+
+// BIG's streamed passes.
+static inline size_t res_vs_bytes(const ResidentPlan& P) {
+#define STREAM(D, SV, NPV, ILV)                             \
+  if (P.dof_n == D && P.slots == SV && P.passes == NPV)     \
+    return align256(8 * (size_t)P.nblk * RT * SV * (NPV - ResPasses<SV, NPV, ILV>::KEPT));
+  EFEA_RESIDENT(STREAM)
+#undef STREAM
+  return 0;
 }
 
 static inline size_t res_words(const ResidentPlan& P, size_t* halo) {
@@ -931,7 +1041,7 @@ static inline size_t res_words(const ResidentPlan& P, size_t* halo) {
 size_t resident_workspace_bytes(int Nnode, int dof_n, const ResidentPlan& P) {
   const size_t vb = align256(8 * (size_t)Nnode * dof_n), cb = align256(8 * (size_t)P.npiece * res_modes(dof_n));
   size_t halo;
-  return 4 * vb + 2 * cb + res_xp_bytes(P) + align256(8 * res_words(P, &halo)) + align256(sizeof(PcgState));
+  return 4 * vb + 2 * cb + res_xp_bytes(P) + res_vs_bytes(P) + align256(8 * res_words(P, &halo)) + align256(sizeof(PcgState));
 }
 
 static ResWork res_carve(void* ws, int Nnode, int dof_n, const ResidentPlan& P, int64_t* nwords) {
@@ -945,6 +1055,7 @@ static ResWork res_carve(void* ws, int Nnode, int dof_n, const ResidentPlan& P, 
   W.z = (double*)c; c += cb;
   W.zs = (double*)c; c += cb;
   W.xp = (double*)c; c += res_xp_bytes(P);
+  W.vs = (double*)c; c += res_vs_bytes(P);
   size_t halo;
   *nwords = (int64_t)res_words(P, &halo);
   W.hx = (u64*)c;
@@ -953,17 +1064,6 @@ static ResWork res_carve(void* ws, int Nnode, int dof_n, const ResidentPlan& P, 
   W.st = (PcgState*)c;
   return W;
 }
-
-// The kernel variants: dof_n, slots per lane, passes, BIG.  A
-// block holds RT / lanes * passes nodes, of at most lanes * slots neighbours
-// each; the largest pass count of each slot count is what 256 registers hold.
-#define EFEA_RESIDENT(X)                                                                    \
-  X(1, 7, 1, false) X(1, 7, 2, false) X(1, 7, 4, false) X(1, 7, 9, true)                     \
-  X(1, 9, 1, false) X(1, 9, 2, false) X(1, 9, 4, false) X(1, 9, 9, true)                     \
-  X(1, 16, 1, false) X(1, 16, 2, false) X(1, 28, 1, false) X(1, 28, 2, false)               \
-  X(2, 4, 1, false) X(2, 4, 2, false) X(2, 4, 4, false)                                     \
-  X(2, 5, 1, false) X(2, 5, 2, false) X(2, 5, 4, false) X(2, 8, 1, false) X(2, 8, 2, false) \
-  X(3, 4, 1, false) X(3, 4, 2, false) X(3, 7, 1, false)
 
 int resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, int* slots, int* passes) {
   int best = 0;
@@ -994,6 +1094,8 @@ static size_t res_lds_bytes(const ResidentPlan& P, int two, int rows) {
 int resident_fits(const ResidentPlan& P) {
   const size_t n = res_lds_bytes(P, P.nagg > 0, 0);
   const int nm = res_modes(P.dof_n), mine = 3 + P.max_pieces * nm, line = (mine + 7) / 8 * 8;
+  // BIG keeps byte offsets of lu's entries in 16 bits
+  if (P.dof_n == 1 && P.passes == 9 && RT * P.passes + P.max_halo > 8191) return 0;
   return n > 0 && n <= (size_t)RES_LDS && P.nblk <= 256 && (P.nagg == 0 || P.ncollect >= 1) && mine <= RT &&
          P.nblk * line <= 65536 && res_columns(P.nagg * nm) <= 32767;
 }
