@@ -77,24 +77,27 @@ __global__ void k_fill_f64(int64_t n, double* __restrict__ a, double v) {
 
 // ---------------------------------------------------------------------------
 // Coarse matrix.  pair_ptr[cb]..pair_ptr[cb+1] lists the (node, neighbour
-// position) pairs whose nodes lie in aggregates (blk_I[cb], blk_J[cb]).
+// position) pairs whose nodes lie in aggregates (blk_I[cb], blk_J[cb]).  A block
+// of eight waves per list: the lists of the diagonal blocks hold most pairs (64^3
+// HEXA8: 14,000 each of 512, in steps of three dependent loads), and with a wave
+// each the chip waited for those (1,522 us; four waves 739, eight 706; 250 x 250
+// TRI3: 66, 28 and 23).
+constexpr int AW = 8;  // waves per list
 template <int DN>
-__global__ void __launch_bounds__(256)
-k_coarse_assemble(int ncb, const int* __restrict__ pair_ptr, const int* __restrict__ pair_node,
+__global__ void __launch_bounds__(64 * AW)
+k_coarse_assemble(const int* __restrict__ pair_ptr, const int* __restrict__ pair_node,
                   const int* __restrict__ pair_pos, const int* __restrict__ blk_I, const int* __restrict__ blk_J,
                   const int* __restrict__ node_ptr, const int* __restrict__ node_cols,
                   const double* __restrict__ vals, const unsigned char* __restrict__ known,
                   const double* __restrict__ rel, double* __restrict__ Ac, int ld) {
-  constexpr int NM = Modes<DN>::NM;
-  const int cb = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (cb >= ncb) return;  // whole wavefront exits together
-  double acc[NM][NM];
+  constexpr int NM = Modes<DN>::NM, N2 = NM * NM, NQ = (N2 + 3) / 4;
+  __shared__ double part[AW][4 * NQ];
+  const int cb = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int k0 = pair_ptr[cb], k1 = pair_ptr[cb + 1];
+  double acc[4 * NQ];
 #pragma unroll
-  for (int m = 0; m < NM; ++m)
-#pragma unroll
-    for (int l = 0; l < NM; ++l) acc[m][l] = 0;
-  for (int k = pair_ptr[cb] + lane; k < pair_ptr[cb + 1]; k += 64) {
+  for (int m = 0; m < 4 * NQ; ++m) acc[m] = 0;
+  for (int k = k0 + threadIdx.x; k < k1; k += 64 * AW) {
     const int i = pair_node[k], pos = pair_pos[k];
     const int p0 = node_ptr[i], cnt = node_ptr[i + 1] - p0;
     const int j = node_cols[p0 + pos];
@@ -118,25 +121,25 @@ k_coarse_assemble(int ncb, const int* __restrict__ pair_ptr, const int* __restri
       for (int m = 0; m < NM; ++m) {
         const double pm = pmode<DN>(ri, a, m);
 #pragma unroll
-        for (int l = 0; l < NM; ++l) acc[m][l] += pm * T[l];
+        for (int l = 0; l < NM; ++l) acc[m * NM + l] += pm * T[l];
       }
     }
   }
+  const int waves = (k1 - k0 + 63) / 64;  // waves with a pair of their own
+  if (wv < waves) {
 #pragma unroll
-  for (int m = 0; m < NM; ++m)
-#pragma unroll
-    for (int l = 0; l < NM; ++l) {
-      double v = acc[m][l];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-      acc[m][l] = v;
+    for (int m = 0; m < NQ; ++m) {
+      const double v = wave_sum4(acc[4 * m], acc[4 * m + 1], acc[4 * m + 2], acc[4 * m + 3]);
+      const int row = lane >> 4, e = row == 1 ? 2 : (row == 2 ? 1 : row);
+      if ((lane & 15) == 0) part[wv][4 * m + e] = v;
     }
-  if (lane == 0) {
-    const int I = blk_I[cb], J = blk_J[cb];
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-      for (int l = 0; l < NM; ++l) Ac[(int64_t)(I * NM + m) * ld + J * NM + l] = acc[m][l];
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < N2) {
+    double v = 0;
+    for (int w = 0; w < (waves < AW ? waves : AW); ++w) v += part[w][t];
+    Ac[(int64_t)(blk_I[cb] * NM + t / NM) * ld + blk_J[cb] * NM + t % NM] = v;
   }
 }
 
@@ -161,96 +164,136 @@ __global__ void k_coarse_guard(int ld, double* __restrict__ Ac, double shift) {
 // (final once the update of step k is done) share one launch: two launches
 // per block step.
 
-// Wavefront broadcast of lane `lane`'s value (lane is a compile-time constant
-// after unrolling).
-__device__ inline double readlane_f64(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Inverts pivot block k with the first wavefront of the block: lane l < GB
-// holds row l in registers; each elimination step broadcasts the pivot row
-// with readlane (no LDS, no barrier).  Writes P to Pb and in place.
-__device__ inline void gj_pivot_wave(double* __restrict__ A, int ld, int k, double* __restrict__ Pb) {
-  const int l = threadIdx.x;
-  if (l >= 64) return;
-  const int k0 = k * GB;
-  const bool own = l < GB;
-  double row[GB];
+// Inverts pivot block k with a block of 256 threads: thread (r, q) holds four
+// columns of row r, and two pivot rows and columns at a time pass through LDS
+// (two buffers in turn, one barrier), the second as the first's elimination
+// leaves it.  A chain of LDS round trips, barriers and divisions; one wave that
+// broadcast each row lane by lane took 13.6 us, this one 9.7 (one elimination per
+// exchange in unrolled code: 9.4 to 9.8).  Writes P to Pb and in place.
+struct PivotLds {
+  double row[2][2][GB], col[2][2][GB];
+};
+__device__ inline void gj_pivot(double* __restrict__ A, int ld, int k, double* __restrict__ Pb, PivotLds& S) {
+  const int r = threadIdx.x % GB, c0 = threadIdx.x / GB * 4;
+  double* a = A + (int64_t)(k * GB + r) * ld + k * GB + c0;
+  double v[4];
 #pragma unroll
-  for (int j = 0; j < GB; ++j) row[j] = own ? A[(int64_t)(k0 + l) * ld + k0 + j] : 0.0;
+  for (int j = 0; j < 4; ++j) v[j] = a[j];
+  // not unrolled further: the loop fits the instruction cache, 32 steps' code is
+  // fetched anew in every launch
+#pragma unroll 1
+  for (int g = 0; g < GB; g += 4)
 #pragma unroll
-  for (int s = 0; s < GB; ++s) {
-    double rs[GB];
+  for (int h = 0; h < 4; h += 2) {
+    const int s = g + h, u = s + 1, buf = h / 2;
+    if (r == s || r == u) {
 #pragma unroll
-    for (int j = 0; j < GB; ++j) rs[j] = readlane_f64(row[j], s);
-    const double p = 1.0 / rs[s];
-    const double ap = row[s] * p;
-    const bool piv = l == s;
+      for (int j = 0; j < 4; ++j) S.row[buf][r - s][c0 + j] = v[j];
+    }
+    if (c0 == g) {
+      S.col[buf][0][r] = v[h];
+      S.col[buf][1][r] = v[h + 1];
+    }
+    __syncthreads();
+    // elimination s, of this row's entries and of what the next one reads
+    const double us = S.row[buf][1][s], su = S.row[buf][0][u];
+    const double p = 1.0 / S.row[buf][0][s], m = S.col[buf][0][r] * p, mu = us * p;
+    // elimination u, with row u and column u as s leaves them
+    const double pu = 1.0 / (S.row[buf][1][u] - mu * su);
+    const double cu = r == s ? su * p : S.col[buf][1][r] - m * su, n = cu * pu;
 #pragma unroll
-    for (int j = 0; j < GB; ++j) {
-      const double upd = (j == s) ? -ap : row[j] - ap * rs[j];
-      const double prow = (j == s) ? p : rs[j] * p;
-      row[j] = piv ? prow : upd;
+    for (int j = 0; j < 4; ++j) {
+      const int cj = c0 + j;
+      const double w = S.row[buf][0][cj];
+      double x = cj == s ? -m : v[j] - m * w;
+      if (r == s) x = cj == s ? p : w * p;
+      const double wu = cj == s ? -mu : S.row[buf][1][cj] - mu * w;
+      double y = cj == u ? -n : x - n * wu;
+      if (r == u) y = cj == u ? pu : wu * pu;
+      v[j] = y;
     }
   }
-  if (own) {
 #pragma unroll
-    for (int j = 0; j < GB; ++j) {
-      Pb[l * GB + j] = row[j];
-      A[(int64_t)(k0 + l) * ld + k0 + j] = row[j];
-    }
+  for (int j = 0; j < 4; ++j) {
+    Pb[r * GB + c0 + j] = v[j];
+    a[j] = v[j];
   }
 }
 
-__global__ void __launch_bounds__(64) k_gj_pivot(double* __restrict__ A, int ld, int k, double* __restrict__ Pb) {
-  gj_pivot_wave(A, ld, k, Pb);
+__global__ void __launch_bounds__(256) k_gj_pivot(double* __restrict__ A, int ld, int k, double* __restrict__ Pb) {
+  __shared__ PivotLds S;
+  gj_pivot(A, ld, k, Pb, S);
 }
 
-// Trailing update of tile (i, j), i, j != k: A_ij -= A_ik (P A_kj) with the
-// row panel unscaled (PRESCALED false: the tile forms P A_kj itself) or
-// A_ij -= A_ik A_kj with the row panel already scaled (PRESCALED true).
+// One 16 x 16 quarter of a product of two GB x GB tiles on the FP64 matrix
+// cores (the layout of elements_mfma.hip): lane l feeds row or column l % 16 and
+// one entry of the sum per step, here 8 (l / 16) + t, so that a lane of the left
+// operand reads 64 bytes in a row, and holds rows 4 v + l / 16, column l % 16 of
+// the result.  With the left operand's rows taken in the order of `mix` those
+// are entries 8 (l / 16) + v (+ 4 with h = 1): a product's two quarters of a
+// column are the right operand of the next product as they are.
+typedef double d4 __attribute__((ext_vector_type(4)));
+struct Left {   // 16 rows of a tile
+  double v[GB / 4];
+  __device__ Left(const double* a, int ld, int row) {
+    const double* p = a + (int64_t)row * ld + 8 * ((threadIdx.x & 63) >> 4);
+#pragma unroll
+    for (int t = 0; t < GB / 4; ++t) v[t] = p[t];
+  }
+};
+struct Right {  // 16 columns of a tile
+  double v[GB / 4];
+  __device__ Right(const double* a, int ld) {
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int t = 0; t < GB / 4; ++t) v[t] = a[(int64_t)(8 * (l >> 4) + t) * ld + (l & 15)];
+  }
+};
+__device__ inline int mix(int h) {
+  const int i = threadIdx.x & 15;
+  return 8 * (i % 4) + i / 4 + 4 * h;
+}
+__device__ inline d4 quarter(const Left& L, const Right& R) {
+  d4 acc = {0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < GB / 4; ++t) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(L.v[t], R.v[t], acc, 0, 0, 0);
+  return acc;
+}
+
+// Trailing update of tile (i, j), i, j != k, a wave per quarter: A_ij -= A_ik
+// (P A_kj) with the row panel unscaled (PRESCALED false: the tile forms P A_kj
+// itself) or A_ij -= A_ik A_kj with the row panel already scaled (PRESCALED
+// true).  Bound by the panels' way from another XCD's L2: 8 x 8 tiles 4.4 us a
+// step, 24 x 24 7.7 (8.0 and 16 with the products through LDS; 12.0 with operands
+// of 32 bytes per row).
 template <bool PRESCALED>
 __global__ void __launch_bounds__(256) k_gj_update(double* __restrict__ A, int ld, int n, int k,
                                                    const double* __restrict__ Pb) {
-  __shared__ double Ps[GB][GB + 1];
-  __shared__ double L[GB][GB + 1];
-  __shared__ double R[GB][GB + 1];
-  __shared__ double T[GB][GB + 1];
   const int nbk = n / GB;
   int ib = blockIdx.y, jb = blockIdx.x;
   if (ib >= k) ++ib;
   if (jb >= k) ++jb;
   if (ib >= nbk || jb >= nbk) return;
-  const int k0 = k * GB, i0 = ib * GB, j0 = jb * GB;
-  for (int e = threadIdx.x; e < GB * GB; e += 256) {
-    const int r = e / GB, c = e % GB;
-    if (!PRESCALED) Ps[r][c] = Pb[e];
-    L[r][c] = A[(int64_t)(i0 + r) * ld + k0 + c];
-    R[r][c] = A[(int64_t)(k0 + r) * ld + j0 + c];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < GB * GB; e += 256) {
-    const int r = e / GB, c = e % GB;
-    double s = 0;
-    if (PRESCALED) {
-      s = R[r][c];
-    } else {
-#pragma unroll 8
-      for (int t = 0; t < GB; ++t) s += Ps[r][t] * R[t][c];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int i0 = ib * GB + 16 * (w >> 1), j0 = jb * GB + 16 * (w & 1), k0 = k * GB;
+  const Left L(A + (int64_t)i0 * ld + k0, ld, l & 15);
+  Right R(A + (int64_t)k0 * ld + j0, ld);
+  double* a = A + (int64_t)(i0 + (l >> 4)) * ld + j0 + (l & 15);
+  double old[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) old[v] = a[(int64_t)4 * v * ld];
+  if constexpr (!PRESCALED) {
+    const Left P0(Pb, GB, mix(0)), P1(Pb, GB, mix(1));
+    const d4 t0 = quarter(P0, R), t1 = quarter(P1, R);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      R.v[v] = t0[v];
+      R.v[4 + v] = t1[v];
     }
-    T[r][c] = s;
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < GB * GB; e += 256) {
-    const int r = e / GB, c = e % GB;
-    double s = 0;
-#pragma unroll 8
-    for (int t = 0; t < GB; ++t) s += L[r][t] * T[t][c];
-    A[(int64_t)(i0 + r) * ld + j0 + c] -= s;
-  }
+  const d4 u = quarter(L, R);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) a[(int64_t)4 * v * ld] = old[v] - u[v];
 }
 
 // Panels of step k and the inversion of pivot block k+1.  WHICH 0: blocks
@@ -259,38 +302,27 @@ __global__ void __launch_bounds__(256) k_gj_update(double* __restrict__ A, int l
 template <int WHICH>
 __global__ void __launch_bounds__(256) k_gj_panels(double* __restrict__ A, int ld, int n, int k,
                                                    const double* __restrict__ Pb, double* __restrict__ Pnext) {
-  __shared__ double Ps[GB][GB + 1];
-  __shared__ double T[GB][GB + 1];
+  __shared__ PivotLds S;
   const int nbk = n / GB;
   const int nrow = WHICH == 2 ? 0 : nbk - 1, ncol = WHICH == 1 ? 0 : nbk - 1;
   const int b = blockIdx.x;
   if (b >= nrow + ncol) {
-    if (WHICH != 1 && k + 1 < nbk) gj_pivot_wave(A, ld, k + 1, Pnext);
+    if (WHICH != 1 && k + 1 < nbk) gj_pivot(A, ld, k + 1, Pnext, S);
     return;
   }
   const bool rowp = b < nrow;
   int t = rowp ? b : b - nrow;
   if (t >= k) ++t;
-  const int k0 = k * GB, t0 = t * GB;
-  for (int e = threadIdx.x; e < GB * GB; e += 256) {
-    const int r = e / GB, c = e % GB;
-    Ps[r][c] = Pb[e];
-    T[r][c] = rowp ? A[(int64_t)(k0 + r) * ld + t0 + c] : A[(int64_t)(t0 + r) * ld + k0 + c];
-  }
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  double* tile = A + (rowp ? (int64_t)k * GB * ld + t * GB : (int64_t)t * GB * ld + k * GB);
+  const Left L(rowp ? Pb + 16 * (w >> 1) * GB : tile + (int64_t)16 * (w >> 1) * ld, rowp ? GB : ld, l & 15);
+  const Right R(rowp ? tile + 16 * (w & 1) : Pb + 16 * (w & 1), rowp ? ld : GB);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every quarter has read the tile
   __syncthreads();
-  for (int e = threadIdx.x; e < GB * GB; e += 256) {
-    const int r = e / GB, c = e % GB;
-    double s = 0;
-    if (rowp) {
-#pragma unroll 8
-      for (int q = 0; q < GB; ++q) s += Ps[r][q] * T[q][c];
-      A[(int64_t)(k0 + r) * ld + t0 + c] = s;
-    } else {
-#pragma unroll 8
-      for (int q = 0; q < GB; ++q) s += T[r][q] * Ps[q][c];
-      A[(int64_t)(t0 + r) * ld + k0 + c] = -s;
-    }
-  }
+  const d4 u = quarter(L, R);
+  double* a = tile + (int64_t)(16 * (w >> 1) + (l >> 4)) * ld + 16 * (w & 1) + (l & 15);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) a[(int64_t)4 * v * ld] = rowp ? u[v] : -u[v];
 }
 
 // X <- (X + X^T) / 2 (upper triangle pairs).
@@ -309,7 +341,7 @@ __global__ void k_symmetrize(double* __restrict__ A, int ld) {
 // inverses used in turn).
 static void gj_invert(double* A, int ld, int n, double* Pb, hipStream_t s) {
   const int nbk = n / GB;
-  hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(64), 0, s, A, ld, 0, Pb);
+  hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(256), 0, s, A, ld, 0, Pb);
   for (int k = 0; k < nbk; ++k) {
     double* Pk = Pb + (k & 1) * GB * GB;
     double* Pn = Pb + ((k + 1) & 1) * GB * GB;
@@ -385,8 +417,8 @@ static int coarse_setup_t(int ncb, const int* pair_ptr, const int* pair_node, co
   const int64_t n2 = (int64_t)ld * ld;
   hipLaunchKernelGGL(k_fill_f64, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, s, n2, Ac, 0.0);
   if (ncb > 0)
-    hipLaunchKernelGGL((k_coarse_assemble<DN>), dim3((unsigned)((ncb + 3) / 4)), dim3(256), 0, s, ncb, pair_ptr,
-                       pair_node, pair_pos, blk_I, blk_J, node_ptr, node_cols, vals, known, rel, Ac, ld);
+    hipLaunchKernelGGL((k_coarse_assemble<DN>), dim3((unsigned)ncb), dim3(64 * AW), 0, s, pair_ptr, pair_node,
+                       pair_pos, blk_I, blk_J, node_ptr, node_cols, vals, known, rel, Ac, ld);
   hipLaunchKernelGGL(k_coarse_guard, dim3((unsigned)((ld + 255) / 256)), dim3(256), 0, s, ld, Ac, shift);
   if (ld > GJ_BLAS_MIN) {
     if (int e = gj_invert_blocked(Ac, ld, Pb, s)) return e;

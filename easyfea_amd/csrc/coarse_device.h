@@ -8,6 +8,52 @@
 
 namespace efea {
 
+// Wave sums of four values at once: the halves of two values change places
+// (v_permlane32_swap: lanes 0-31 then hold the one, 32-63 the other), then the
+// rows of two such pairs (v_permlane16_swap), which leaves one value per row of
+// 16 lanes and a rotation sum within the row: 7 additions for four values.  A
+// butterfly of __shfl_xor takes 24 and an LDS round trip each.  Row 0 gets a's
+// sum, row 1 c's, row 2 b's, row 3 d's, in all 16 lanes.
+__device__ inline double join64(unsigned lo, unsigned hi) {
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <bool ROW16>
+__device__ inline double swap_add(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  if constexpr (ROW16) {
+    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return join64(l[0], h[0]) + join64(l[1], h[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return join64(l[0], h[0]) + join64(l[1], h[1]);
+  }
+}
+template <int ROR>
+__device__ inline double ror_add(double v) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)x, 0x120 + ROR, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), 0x120 + ROR, 0xf, 0xf, true);
+  return v + join64(lo, hi);
+}
+__device__ inline double wave_sum4(double a, double b, double c, double d) {
+  double v = swap_add<true>(swap_add<false>(a, b), swap_add<false>(c, d));
+  v = ror_add<8>(v);
+  v = ror_add<4>(v);
+  v = ror_add<2>(v);
+  return ror_add<1>(v);
+}
+// One value's sum, in every lane.
+__device__ inline double wave_sum1(double v) {
+  v = swap_add<false>(v, v);
+  v = swap_add<true>(v, v);
+  v = ror_add<8>(v);
+  v = ror_add<4>(v);
+  v = ror_add<2>(v);
+  return ror_add<1>(v);
+}
+
 // Rigid-body mode m of DOF component a at a node with coordinates r relative
 // to its aggregate centroid.
 template <int DN>
