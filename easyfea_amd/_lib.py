@@ -44,6 +44,8 @@ SIGNATURES = {
         [i32, i32, vp, i32, vp, vp, vp, vp, vp, vp, i32, vp, i32, f64, i32, f64, vp, i32, vp, vp],
     ),
     "efea_assemble_max_neighbours": (i32, [i32]),
+    "efea_row_counts": (i32, [i32, i32, vp, vp, vp, vp, vp]),
+    "efea_row_plan": (i32, [i32, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
     "efea_elastic_strain_stress": (i32, [i32, i64, vp, vp, vp, i32, vp, vp, i32, f64, i32, f64, vp, vp]),
     "efea_node_average": (i32, [i32, i32, vp, vp, vp, vp, vp]),
     "efea_csr_scatter": (i32, [i32, i64, vp, vp, vp, vp, vp]),

@@ -31,6 +31,68 @@
 
 namespace efea {
 
+// The plan of the assembly by rows, from the scatter map: the entries that a
+// node's own (diagonal) slot sums are its incidences, elements increasing.
+__device__ inline int place(const int* __restrict__ cols, int p0, int p1, int j) {
+  int lo = p0, hi = p1 - 1;  // j is in the row
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (cols[mid] < j) lo = mid + 1; else hi = mid;
+  }
+  return lo - p0;
+}
+__device__ inline int64_t own_slot(const int* __restrict__ node_ptr, const int* __restrict__ node_cols, int dn, int n) {
+  const int p0 = node_ptr[n], p1 = node_ptr[n + 1];
+  return (int64_t)dn * dn * p0 + (p1 > p0 ? dn * place(node_cols, p0, p1, n) : 0);
+}
+
+// counts[n + 1]: the node's incidences (counts[0] = 0).
+__global__ void __launch_bounds__(256) k_row_counts(int Nn, int dn, const int* __restrict__ node_ptr,
+                                                    const int* __restrict__ node_cols, const int* __restrict__ seg,
+                                                    int* __restrict__ counts) {
+  const int n = blockIdx.x * 256 + threadIdx.x;
+  if (n == 0) counts[0] = 0;
+  if (n >= Nn) return;
+  const int64_t s = own_slot(node_ptr, node_cols, dn, n);
+  counts[n + 1] = node_ptr[n + 1] > node_ptr[n] ? seg[s + 1] - seg[s] : 0;
+}
+
+// A wave per node, a lane per (incidence, element node).  repeated: set where an
+// element names a node twice.
+__global__ void __launch_bounds__(64) k_row_plan(int dn, int nPe, const int* __restrict__ node_ptr,
+                                                 const int* __restrict__ node_cols, const int* __restrict__ seg,
+                                                 const int* __restrict__ perm, const int* __restrict__ connect,
+                                                 const int* __restrict__ inc_ptr, int* __restrict__ inc,
+                                                 unsigned short* __restrict__ pos, int* __restrict__ repeated) {
+  const int n = blockIdx.x, nd = nPe * dn;
+  const int p0 = node_ptr[n], p1 = node_ptr[n + 1], i0 = inc_ptr[n], num = inc_ptr[n + 1] - i0;
+  if (num <= 0) return;
+  const int first = seg[own_slot(node_ptr, node_cols, dn, n)];
+  for (int q = threadIdx.x; q < num * nPe; q += 64) {
+    const int k = q / nPe, lj = q % nPe, entry = perm[first + k];
+    const int e = entry / (nd * nd), li = entry % (nd * nd) / nd / dn;
+    if (lj == 0) {
+      inc[i0 + k] = e * 16 + li;
+      if (entry % nd / dn != li) *repeated = 1;
+    }
+    pos[(int64_t)(i0 + k) * nPe + lj] = (unsigned short)place(node_cols, p0, p1, connect[(int64_t)e * nPe + lj]);
+  }
+}
+
+int row_counts(int Nn, int dof_n, const int* node_ptr, const int* node_cols, const int* seg, int* counts,
+               hipStream_t s) {
+  hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((Nn + 255) / 256)), dim3(256), 0, s, Nn, dof_n, node_ptr, node_cols,
+                     seg, counts);
+  return check_launch("row_counts");
+}
+
+int row_plan(int Nn, int dof_n, int nPe, const int* node_ptr, const int* node_cols, const int* seg, const int* perm,
+             const int* connect, const int* inc_ptr, int* inc, unsigned short* pos, int* repeated, hipStream_t s) {
+  hipLaunchKernelGGL(k_row_plan, dim3((unsigned)Nn), dim3(64), 0, s, dof_n, nPe, node_ptr, node_cols, seg, perm,
+                     connect, inc_ptr, inc, pos, repeated);
+  return check_launch("row_plan");
+}
+
 // LDS a block may use for its rows (the groups' 8 KB at most come on top): three
 // blocks on a CU.  Longer rows than this allows (HEXA8: 85 nodes, TETRA10: 170)
 // go through element matrices.

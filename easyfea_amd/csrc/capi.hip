@@ -115,6 +115,9 @@ int pp_iter_bench(int, int, int, int, const int*, const int*, const double*, con
                   hipStream_t);
 
 int assemble_max_neighbours(int);
+int row_counts(int, int, const int*, const int*, const int*, int*, hipStream_t);
+int row_plan(int, int, int, const int*, const int*, const int*, const int*, const int*, const int*, int*,
+             unsigned short*, int*, hipStream_t);
 int elastic_assemble(int, int, const int*, int, const int*, const int*, const unsigned short*, const int*,
                      const double*, const double*, int, const double*, int, double, int, double, const double*, int,
                      double*, hipStream_t);
@@ -193,6 +196,27 @@ int efea_elastic_ke_dense(int elem_type, int64_t Ne, const int32_t* connect, con
 }
 
 int efea_assemble_max_neighbours(int elem_type) { return assemble_max_neighbours(elem_type); }
+
+int efea_row_counts(int Nn, int dof_n, const int32_t* node_ptr, const int32_t* node_cols, const int32_t* seg_ptr,
+                    int32_t* counts, void* stream) {
+  if (Nn <= 0 || dof_n < 1 || !node_ptr || !node_cols || !seg_ptr || !counts) {
+    set_error("efea_row_counts: null pointer or empty mesh");
+    return EFEA_ERR_ARG;
+  }
+  return row_counts(Nn, dof_n, node_ptr, node_cols, seg_ptr, counts, STREAM(stream));
+}
+
+int efea_row_plan(int Nn, int dof_n, int nPe, const int32_t* node_ptr, const int32_t* node_cols,
+                  const int32_t* seg_ptr, const int32_t* perm, const int32_t* connect, const int32_t* inc_ptr,
+                  int32_t* inc, uint16_t* pos, int32_t* repeated, void* stream) {
+  if (Nn <= 0 || dof_n < 1 || nPe < 1 || nPe > 16 || !node_ptr || !node_cols || !seg_ptr || !perm || !connect ||
+      !inc_ptr || !inc || !pos || !repeated) {
+    set_error("efea_row_plan: null pointer, empty mesh or more than 16 nodes per element");
+    return EFEA_ERR_ARG;
+  }
+  return row_plan(Nn, dof_n, nPe, node_ptr, node_cols, seg_ptr, perm, connect, inc_ptr, inc, pos, repeated,
+                  STREAM(stream));
+}
 
 int efea_elastic_assemble(int elem_type, int Nn, const int32_t* node_ptr, int max_neighbours, const int32_t* inc_ptr,
                           const int32_t* inc, const uint16_t* pos, const int32_t* connect, const double* coord,

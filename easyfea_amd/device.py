@@ -151,9 +151,23 @@ class DeviceMesh:
         if "row_incidence" not in d:
             p = self.pattern(dof_n)
             fits = p.host.max_neighbours <= _lib.load().efea_assemble_max_neighbours(self.code) and self.Ne < 1 << 27
-            d["row_incidence"] = row_incidence(self.connect, self.Nn, p.node_ptr, p.node_cols) if fits else None
-            torch.cuda.current_stream().synchronize()  # as an upload: any stream may use it from here on
+            d["row_incidence"] = self._row_incidence(p) if fits else None
         return d["row_incidence"]
+
+    def _row_incidence(self, p: "CsrPattern") -> Optional[tuple]:
+        counts = torch.empty(self.Nn + 1, dtype=torch.int32, device="cuda")
+        inc = torch.empty(self.Ne * self.nPe, dtype=torch.int32, device="cuda")
+        pos = torch.empty((self.Ne * self.nPe, self.nPe), dtype=torch.int16, device="cuda")
+        repeated = torch.zeros(1, dtype=torch.int32, device="cuda")
+        _lib.call("efea_row_counts", self.Nn, p.dof_n, ptr(p.node_ptr), ptr(p.node_cols), ptr(p.seg), ptr(counts),
+                  stream_ptr())
+        inc_ptr = counts.cumsum(0, dtype=torch.int32)
+        # a repeated node gives its node more incidences than the lists hold
+        if int(inc_ptr[-1]) != inc.numel():
+            return None
+        _lib.call("efea_row_plan", self.Nn, p.dof_n, self.nPe, ptr(p.node_ptr), ptr(p.node_cols), ptr(p.seg),
+                  ptr(p.perm), ptr(self.connect), ptr(inc_ptr), ptr(inc), ptr(pos), ptr(repeated), stream_ptr())
+        return None if int(repeated) else (inc_ptr, inc, pos)  # the copy to the host waits: any stream may use them
 
     def node_values(self, values_e: torch.Tensor) -> torch.Tensor:
         """Element values (Ne, k) -> node values (Nn, k) (``Mesh.Get_Node_Values``)."""
@@ -188,22 +202,6 @@ class DeviceMesh:
         if dof_n not in v:
             v[dof_n] = DeviceVecMap(build_vec_map(self.connect_np, self.Nn, dof_n))
         return v[dof_n]
-
-
-def row_incidence(connect: torch.Tensor, Nn: int, node_ptr: torch.Tensor, node_cols: torch.Tensor) -> Optional[tuple]:
-    """See ``DeviceMesh.row_incidence`` (torch, on the inputs' device)."""
-    nPe = connect.shape[1]
-    con = connect.long()
-    node, order = torch.sort(con.reshape(-1), stable=True)  # by node, elements increasing
-    e = order // nPe
-    if bool(((node[1:] == node[:-1]) & (e[1:] == e[:-1])).any()):
-        return None
-    nodes = torch.arange(Nn + 1, device=con.device)
-    inc_ptr = torch.searchsorted(node, nodes, out_int32=True)
-    start = node_ptr.long()
-    keys = torch.repeat_interleave(nodes[:-1] * Nn, start[1:] - start[:-1], output_size=len(node_cols)) + node_cols
-    pos = torch.searchsorted(keys, node[:, None] * Nn + con[e]) - start[node][:, None]
-    return inc_ptr, (e * 16 + order % nPe).int(), pos.to(torch.int16)
 
 
 class DeviceVecMap:

@@ -78,6 +78,16 @@ int efea_elastic_assemble(int elem_type, int Nn, const int32_t* node_ptr, int ma
                           const double* tables, int nPg, const double* E, int E_stride, double nu, int plane_stress,
                           double thickness, const double* D, int D_stride, double* values, void* stream);
 int efea_assemble_max_neighbours(int elem_type);
+/* Its plan from the scatter map (seg_ptr, perm of efea_csr_scatter).
+ * efea_row_counts: counts (Nn + 1) = 0, then each node's incidences; their
+ * running sum is inc_ptr.  efea_row_plan fills inc and pos (rows of fewer than
+ * 65536 nodes) and sets *repeated (zeroed by the caller) where an element names
+ * a node twice, which efea_elastic_assemble does not take. */
+int efea_row_counts(int Nn, int dof_n, const int32_t* node_ptr, const int32_t* node_cols, const int32_t* seg_ptr,
+                    int32_t* counts, void* stream);
+int efea_row_plan(int Nn, int dof_n, int nPe, const int32_t* node_ptr, const int32_t* node_cols,
+                  const int32_t* seg_ptr, const int32_t* perm, const int32_t* connect, const int32_t* inc_ptr,
+                  int32_t* inc, uint16_t* pos, int32_t* repeated, void* stream);
 
 /* Linear-elastic post-processing per element (Simulations/_elastic.py:229-380,
  * Models/Elastic/_laws.py:127-185, Models/_utils.py:302-434): at each stiffness

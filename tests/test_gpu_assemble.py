@@ -9,12 +9,11 @@ over the elements of the entry, of each one's largest entry."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
-import torch
 
 import easyfea_amd as ea
 from easyfea_amd import Models, Simulations, _lib
 from easyfea_amd.assembly_map import build_csr_map
-from easyfea_amd.device import row_incidence
+from easyfea_amd.device import DeviceMesh
 from easyfea_amd.mesh import tetra4_box, tetra10_from_tetra4
 from oracle import efea_oracle as O
 
@@ -110,26 +109,33 @@ def test_longest_rows_and_the_ones_beyond():
         assert np.max(np.abs(K - ref) / np.where(size > 0, size, 1.0)) < 1e-14
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dof_n", [1, 2, 3])
 @pytest.mark.parametrize("et", list(MESHES))
-def test_row_incidence_lists_each_pair_once(et):
+def test_row_incidence_lists_each_pair_once(et, dof_n):
     mesh = _mesh(et, 1)
     m = build_csr_map(mesh.connect, mesh.Nn, 1)
-    con = torch.from_numpy(np.ascontiguousarray(mesh.connect))
-    inc_ptr, inc, pos = row_incidence(con, mesh.Nn, torch.from_numpy(m.node_ptr), torch.from_numpy(m.node_cols))
-    nPe = con.shape[1]
-    pos = pos.numpy()
-    assert pos.shape == (con.numel(), nPe) and inc_ptr.dtype == inc.dtype == torch.int32 and pos.dtype == np.int16
-    assert inc_ptr[-1] == con.numel() == len(inc)
+    inc_ptr, inc, pos = (a.cpu().numpy() for a in DeviceMesh(mesh).row_incidence(dof_n))
+    assert inc_ptr[-1] == mesh.connect.size == len(inc) == len(pos)
     for n in range(mesh.Nn):
-        codes = inc[inc_ptr[n]:inc_ptr[n + 1]].numpy()
-        e = codes >> 4
+        rows = slice(inc_ptr[n], inc_ptr[n + 1])
+        e = inc[rows] >> 4
         assert np.all(np.diff(e) > 0)
-        assert np.all(mesh.connect[e, codes & 15] == n)
+        assert np.all(mesh.connect[e, inc[rows] & 15] == n)
         row = m.node_cols[m.node_ptr[n]:m.node_ptr[n + 1]]
-        assert np.array_equal(row[pos[inc_ptr[n]:inc_ptr[n + 1]]], mesh.connect[e])
+        assert np.array_equal(row[pos[rows]], mesh.connect[e])
 
 
-def test_row_incidence_refuses_a_repeated_node():
-    con = torch.tensor([[0, 1, 2, 3], [1, 4, 4, 2]], dtype=torch.int32)
-    m = build_csr_map(con.numpy(), 5, 1)
-    assert row_incidence(con, 5, torch.from_numpy(m.node_ptr), torch.from_numpy(m.node_cols)) is None
+@pytest.mark.gpu
+def test_a_repeated_node_keeps_element_matrices():
+    """A QUAD4 mesh whose last element is collapsed to a triangle."""
+    mesh = ea.quad4_rectangle(3.0, 2.0, 4, 3)
+    con = mesh.connect.copy()
+    con[-1, 3] = con[-1, 2]
+    mesh = ea.Mesh({"QUAD4": con}, mesh.coord)
+    law = Models.Elastic.Isotropic(2, 210000.0, 0.3)
+    simu = Simulations.Elastic(mesh, law)
+    K = simu.Assembly().to_scipy().toarray()
+    assert simu.dev.row_incidence(2) is None
+    ref, size = _reference(mesh, "QUAD4", O.C_isotropic(210000.0, 0.3, 2, law.planeStress), law.thickness)
+    assert np.max(np.abs(K - ref) / np.where(size > 0, size, 1.0)) < 1e-14
