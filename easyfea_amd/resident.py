@@ -183,7 +183,8 @@ def neighbours(rows: torch.Tensor, node_ptr: torch.Tensor, node_cols: torch.Tens
     local[cross] = nloc + place - halo_ptr[brow[cross]]
     if lanes == 1:  # scalar rows: the node itself first, without an entry
         own = node_cols.long() == row
-        self_k = k[own]
+        self_k = torch.zeros(Nn, dtype=k.dtype, device=dev)  # a node of no element has an empty row
+        self_k[row[own]] = k[own]
         k = torch.where(own, 0, torch.where(k < self_k[row], k + 1, k))
     per = 64 // lanes
     p = prow % nloc
