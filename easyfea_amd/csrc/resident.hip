@@ -316,7 +316,9 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     const bool have = nd >= 0;
     const int n = have ? nd : 0;
     const int p0 = A.node_ptr[n], cnt = A.node_ptr[n + 1] - p0;
-    const int64_t base = (int64_t)DN * DN * p0;
+    // a node of no element has an empty row: its loads (dropped) go to the first
+    // values, where p0 of a last such node would be past the end
+    const int64_t base = cnt > 0 ? (int64_t)DN * DN * p0 : 0;
     const int self = DN == 1 ? P.self[gp] : 0;
     double* vs = W.vs + ((int64_t)blk * (NP - NV) + (p - NV)) * S * RT + t;  // a streamed pass
 #pragma unroll
