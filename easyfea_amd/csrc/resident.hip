@@ -759,6 +759,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int nd = BIG ? P.rows[(int64_t)blk * NLOC + at(p)] : node[BIG ? 0 : p];
+      if constexpr (BIG) lu[at(p)] = 0.0;  // a position without a node enters the sums too
       if (nd >= 0 && own) {
         const int64_t i = (int64_t)nd * DN + g;
         rv[p] = W.r[i];

@@ -115,6 +115,25 @@ def test_paused_solve_continues_bit_for_bit(case):
         assert (info.iterations, info.rel_residual, info.status) == (wi.iterations, wi.rel_residual, 1)
 
 
+def test_continued_solve_does_not_depend_on_what_ran_between():
+    """The 9-pass variant: between the start and the finish, a solve of NaN on
+    a system that fills its blocks leaves NaN in the LDS of the CUs, at the
+    positions where the continued solve's blocks hold no node as well."""
+    A, b, x0, known = _system(Q(1, 1, 730, 720), 1)
+    B, c, y0, knownB = _system(Q(1, 1, 683, 767), 1)  # 114 blocks of 4608 nodes
+    whole, wi = _run(A, b, x0, known, "bj", "auto")
+    p = whole.resident.plan
+    assert (p.slots, p.passes) == (9, 9) and p.nblk * 4608 > A.Nn
+    y0.fill_(float("nan"))  # the last product is that of x
+    job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond="bj", expected_iterations=9)
+    pending = job.start()
+    _run(B, c, y0, knownB, "bj", "auto")
+    assert B.pattern.resident().plan.nblk * 4608 == B.Nn
+    info = pending.finish()
+    assert pending.resumed and info.resident and not info.fallback
+    assert torch.equal(job.x, whole.x) and info.iterations == wi.iterations
+
+
 def test_a_block_that_waits_too_long_gives_up(monkeypatch):
     """A wait limit no exchange can meet: the solve fails, every wait ends, and
     the classic iteration redoes it from the same start."""
