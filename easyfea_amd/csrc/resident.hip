@@ -321,6 +321,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     const int64_t base = cnt > 0 ? (int64_t)DN * DN * p0 : 0;
     const int self = DN == 1 ? P.self[gp] : 0;
     double* vs = W.vs + ((int64_t)blk * (NP - NV) + (p - NV)) * S * RT + t;  // a streamed pass
+    bool diag = false, off = false;  // BIG: not zero
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       int j = g + s * G;
@@ -338,6 +339,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
             vs[s * RT] = ok ? vv : 0.0;
             if (s == 0) dg[p - NV] = ok ? vv : 0.0;
           }
+          if (BIG && ok && vv != 0.0) (s == 0 ? diag : off) = true;
         }
     }
     if constexpr (!BIG) {
@@ -364,6 +366,13 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     if (kn) kmask |= 1u << p;
     rv[p] = sv[p] = 0.0;
     if constexpr (BIG) {
+      // A row of zeros keeps its x, as it does with efea_bj_setup's 1 in place of
+      // the zero diagonal.  Where only the diagonal is zero, or b is not, the
+      // solve breaks down at once and the classic iteration takes it.
+      if (!kn && !diag) {
+        kmask |= 1u << p;
+        if (off || !(A.b[i] == 0.0)) rv[p] = __longlong_as_double(0x7ff8000000000000ll);
+      }
       lp[at(p)] = 0.0;
     } else {
       node[p] = nd;

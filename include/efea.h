@@ -450,7 +450,9 @@ int efea_resident_shape(int dof_n, int max_neighbours, int min_passes, int* lane
 /* 1 if a block of the plan (sizes only; the pointers are not read) fits a CU's LDS. */
 int efea_resident_fits(const efea_resident_plan* plan);
 size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan);
-/* The solve; Minv FP64 (efea_bj_setup), rel / Ainv / ld as in efea_solve_pcg2
+/* The solve; Minv FP64, the inverse efea_bj_setup makes (plans of nine passes,
+ * dof_n 1, form it from the diagonal instead and break down at an unknown row of
+ * zero diagonal, unless the row and b are 0 there), rel / Ainv / ld as in efea_solve_pcg2
  * (ignored without aggregates), info as in efea_solve_pcg.  A block waits at
  * most wait_ms (<= 0: 250) for the others; a solve given up so, a refused
  * launch and a breakdown return EFEA_ERR_NOCONV with status 2, and the caller

@@ -160,6 +160,29 @@ def test_zero_and_non_finite_right_hand_sides(dof_n, precond):
         assert info.status == 2
 
 
+@pytest.mark.parametrize("cells", [(40, 40), (730, 720)])  # one pass, nine
+def test_an_unknown_row_of_zeros(cells):
+    """block Jacobi puts 1 in place of a zero diagonal: the row stays at its start."""
+    A, b, x0, known = _system(Q(1, 1, *cells), 1)
+    n = A.Nn // 2
+    at = torch.nonzero(A.pattern.node_cols == n).flatten()
+    A.values[at] = 0.0
+    A.values[int(A.node_ptr[n]):int(A.node_ptr[n + 1])] = 0.0
+    b[n], x0[n] = 0.0, 0.25
+    assert not known[n]
+    job, info = _run(A, b, x0, known, "bj", "auto")
+    assert job.resident.plan.passes == (1 if cells[0] == 40 else 9)
+    assert info.status == 1 and info.resident and not info.fallback
+    classic, _ = _run(A, b, x0, known, "bj", False)
+    assert float(job.x[n]) == float(classic.x[n]) == 0.25
+    assert _close(job.x, classic.x, known) < 1e-8
+    b[n] = 1.0  # no solution
+    for pipelined in ("auto", False):
+        job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond="bj", pipelined=pipelined, maxit=300)
+        info = job.run(raise_on_fail=False)
+        assert info.status != 1
+
+
 def test_two_threads_on_their_own_streams():
     """Solves of two threads at once take the chip in turn, with the results of
     one after the other."""
