@@ -684,9 +684,10 @@ class SolveJob:
 
     def _wants_resident(self) -> Optional[Resident]:
         """The plan of a resident solve: FP64, unless the caller asked for the
-        classic iteration, whatever the expected count (its recurrences do not
-        drift), wherever the matrix fits the chip's registers."""
-        if self.pipelined_mode is False or self.precision != 64 or self.method != "pcg":
+        classic iteration or a cap on the solver kernels' grids (a plan takes
+        the blocks it needs), whatever the expected count (its recurrences do
+        not drift), wherever the matrix fits the chip's registers."""
+        if self.pipelined_mode is False or self.precision != 64 or self.method != "pcg" or self.max_blocks > 0:
             return None
         if self.precond == "two-level":
             return self.A.pattern.resident(self.A.coarse(self.coarse_target))

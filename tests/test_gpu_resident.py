@@ -214,6 +214,22 @@ def test_two_threads_on_their_own_streams():
             assert resident and torch.equal(x, want[k])
 
 
+@pytest.mark.parametrize("precond", ["bj", "two-level"])
+def test_a_grid_cap_keeps_the_launch_per_step_iteration(precond):
+    A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
+
+    def run(max_blocks, pipelined):
+        job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond=precond, max_blocks=max_blocks,
+                          pipelined=pipelined)
+        return job, job.run()
+
+    job, info = run(3, "auto")
+    assert info.status == 1 and not info.resident and not info.fallback
+    if precond == "bj":  # the cap is part of the order of the sums
+        assert torch.equal(job.x, run(3, False)[0].x)
+    assert run(0, "auto")[1].resident
+
+
 def test_refused_arguments():
     lib = _lib.load()
     fake, info = 0x1000, (C.c_double * 4)()
