@@ -714,7 +714,7 @@ int pcg_finish_info(const void* state, double rr_true, double* info);
 struct PollBuf {
   PcgState st;
   double rr;
-  int failed;  // resident solve: a block gave up waiting for another
+  int failed;  // resident solve: 1 a block gave up waiting for another, 2 not launched
 };
 PollBuf* poll_buffer(int slot = 0);
 // Phases of the pipelined block-Jacobi solve (solve_pcgp): the whole solve,

@@ -1194,7 +1194,7 @@ int solve_resident(const ResidentPlan& P, int Nnode, const int* node_ptr, const 
     if (phase == PCGP_START) {
       if (e == EFEA_ERR_NOCONV) {  // the finish reports it
         if (hipStreamSynchronize(s) != hipSuccess) return EFEA_ERR_HIP;
-        pb->failed = 1;
+        pb->failed = 2;
         return 0;
       }
       return e;
@@ -1215,8 +1215,11 @@ int solve_resident(const ResidentPlan& P, int Nnode, const int* node_ptr, const 
     }
   }
   if (pb->failed) {
-    set_error("resident: a block waited longer than its limit for another");
-    return refused(EFEA_ERR_NOCONV);
+    set_error(pb->failed == 1 ? "resident: a block waited longer than its limit for another"
+                              : "resident: the launch of %d blocks was refused", P.nblk);
+    refused(EFEA_ERR_NOCONV);
+    info[2] = pb->failed == 1;
+    return EFEA_ERR_NOCONV;
   }
   const PcgState fin = pb->st;
   return pcg_finish_info(&fin, pb->rr, info);

@@ -8,6 +8,8 @@ without a GPU the constructors raise.
 from __future__ import annotations
 
 import ctypes as C
+import threading
+import time
 from dataclasses import dataclass
 from typing import Callable, Optional
 
@@ -536,6 +538,42 @@ PIPELINE_BJ_MAX_EXPECTED = 128
 # Longest wait of a resident solve's block for another one before the solve is
 # given up and redone with the classic iteration (0: the library's 250 ms).
 RESIDENT_WAIT_MS = 0.0
+
+
+class ResidentPauses:
+    """Where blocks of a resident solve cannot all be on the chip together (a
+    program that shares the device, a stream that holds CUs for long), each
+    solve would wait out its limit before it is redone: 250 ms for a solve of
+    one.  After two given up in a row on a device its solves therefore take the
+    launch-per-step iterations for FIRST seconds, then one tries again; while
+    they fail the pause doubles, up to MOST, so that waits stay below an eighth
+    of the time, and far below it as it lasts.  One that succeeds ends it."""
+
+    FIRST, MOST = 2.0, 64.0
+    clock = staticmethod(time.monotonic)
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._row: dict = {}    # device -> solves given up in a row
+        self._until: dict = {}  # device -> end of its pause
+
+    def paused(self, device: int) -> bool:
+        return self._until.get(device, 0.0) > self.clock()
+
+    def gave_up(self, device: int) -> None:
+        with self._lock:
+            row = self._row[device] = self._row.get(device, 0) + 1
+            if row > 1:
+                self._until[device] = self.clock() + min(self.FIRST * 2.0 ** min(row - 2, 30), self.MOST)
+
+    def succeeded(self, device: int) -> None:
+        if device in self._row:
+            with self._lock:
+                self._row.pop(device, None)
+                self._until.pop(device, None)
+
+
+resident_pauses = ResidentPauses()
 # A phase-field displacement solve that stalls with fully damaged nodes is
 # redone with those nodes as singleton aggregates; the attempts before stop
 # after this many iterations (or 4x the previous solve's), the coarse space
@@ -688,6 +726,8 @@ class SolveJob:
         the blocks it needs), whatever the expected count (its recurrences do
         not drift), wherever the matrix fits the chip's registers."""
         if self.pipelined_mode is False or self.precision != 64 or self.method != "pcg" or self.max_blocks > 0:
+            return None
+        if resident_pauses.paused(torch.cuda.current_device()):
             return None
         if self.precond == "two-level":
             return self.A.pattern.resident(self.A.coarse(self.coarse_target))
@@ -864,6 +904,11 @@ class SolveJob:
     def _conclude(self, ws: Workspace, rc: int, si: SolveInfo, raise_on_fail: bool) -> SolveInfo:
         """The fallbacks of a solve that did not converge (see ``run``)."""
         isolating = self.isolate is not None and self.A.pattern.coord is not None
+        if self.resident is not None:
+            if rc == 0:
+                resident_pauses.succeeded(torch.cuda.current_device())
+            elif si.replacements:  # as efea_solve_resident reports a wait given up
+                resident_pauses.gave_up(torch.cuda.current_device())
         if rc != 0 and (self.pipelined or self.resident is not None):
             # a pipelined breakdown (rounding in its recurrences) or a resident
             # solve given up: the classic iteration from the same start
@@ -905,6 +950,8 @@ class SolveJob:
             return None
         ws = ws or Workspace()
         self._prepare()
+        if self.resident is None and not self.pipelined:  # a pause has begun since
+            return None
         if self.before_solve is not None and self.before_solve():
             self._redo_setup()
         check_every, _ = self._polls()

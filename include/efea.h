@@ -454,9 +454,10 @@ size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan);
  * dof_n 1, form it from the diagonal instead and break down at an unknown row of
  * zero diagonal, unless the row and b are 0 there), rel / Ainv / ld as in efea_solve_pcg2
  * (ignored without aggregates), info as in efea_solve_pcg.  A block waits at
- * most wait_ms (<= 0: 250) for the others; a solve given up so, a refused
- * launch and a breakdown return EFEA_ERR_NOCONV with status 2, and the caller
- * redoes the solve from the same start with efea_solve_pcg[2].  The resident
+ * most wait_ms (<= 0: 250) for the others; a solve given up so (info[2] = 1,
+ * else 0: another process may hold a part of the chip), a refused launch and a
+ * breakdown return EFEA_ERR_NOCONV with status 2, and the caller redoes the
+ * solve from the same start with efea_solve_pcg[2].  The resident
  * solves of a process follow one another on a device, also from several
  * streams.  A call waits for the solve, not for what was queued behind it.
  * efea_resident_start / efea_resident_finish are its deferred form, as

@@ -148,6 +148,34 @@ def test_a_block_that_waits_too_long_gives_up(monkeypatch):
     assert info.status == 1 and info.resident
 
 
+def test_solves_given_up_in_a_row_pause_the_resident_route(monkeypatch):
+    """Two given up: none tried for 2 s, then one, and while it fails 4 s."""
+    A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
+    now = [100.0]
+    pauses = dv.ResidentPauses()
+    pauses.clock = lambda: now[0]
+    monkeypatch.setattr(dv, "resident_pauses", pauses)
+
+    def tried():
+        job, info = _run(A, b, x0, known, "two-level", "auto")
+        assert info.status == 1
+        return info.fallback, info.resident
+
+    waits = dv.RESIDENT_WAIT_MS
+    monkeypatch.setattr(dv, "RESIDENT_WAIT_MS", 1e-9)
+    assert [tried() for _ in range(4)] == [(True, False)] * 2 + [(False, False)] * 2
+    now[0] += 2.5
+    assert [tried() for _ in range(2)] == [(True, False), (False, False)]
+    now[0] += 2.5
+    assert tried() == (False, False)
+    job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond="bj", expected_iterations=9)
+    pending = job.start()  # the pipelined form
+    assert pending is not None and pending.entry == "pcgp" and pending.finish().status == 1
+    monkeypatch.setattr(dv, "RESIDENT_WAIT_MS", waits)
+    now[0] += 2.5
+    assert [tried() for _ in range(2)] == [(False, True)] * 2
+
+
 @pytest.mark.parametrize("dof_n,precond", [(1, "bj"), (2, "two-level")])
 def test_zero_and_non_finite_right_hand_sides(dof_n, precond):
     A, b, x0, known = _system(Q(1, 1, 40, 40), dof_n)
