@@ -909,9 +909,11 @@ class SolveJob:
                 resident_pauses.succeeded(torch.cuda.current_device())
             elif si.replacements:  # as efea_solve_resident reports a wait given up
                 resident_pauses.gave_up(torch.cuda.current_device())
-        if rc != 0 and (self.pipelined or self.resident is not None):
+        if rc != 0 and (self.pipelined if self.resident is None else si.status != 0):
             # a pipelined breakdown (rounding in its recurrences) or a resident
-            # solve given up: the classic iteration from the same start
+            # solve given up: the classic iteration from the same start (not
+            # after a resident solve's last iteration: its iterates are the
+            # classic ones, which would end there as well)
             self.pipeline_failure = (rc, _lib.last_error(), si)
             self.x.copy_(self.x0)
             self.pipelined, self.resident = False, None

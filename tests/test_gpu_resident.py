@@ -176,6 +176,24 @@ def test_solves_given_up_in_a_row_pause_the_resident_route(monkeypatch):
     assert [tried() for _ in range(2)] == [(False, True)] * 2
 
 
+@pytest.mark.parametrize("precond", ["bj", "two-level"])
+def test_the_iteration_limit_ends_the_solve(precond):
+    """It is not run again by the classic iteration, which ends at the same iterate."""
+    A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
+    xs = []
+    for pipelined in ("auto", False):
+        job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond=precond, pipelined=pipelined,
+                          maxit=32)
+        info = job.run(raise_on_fail=False)
+        assert (info.status, info.fallback, info.resident) == (0, False, pipelined == "auto")
+        assert info.rel_residual > 1e-6
+        xs.append((job.x, info.iterations))
+    assert xs[0][1] == xs[1][1]
+    assert _close(xs[0][0], xs[1][0], known) < 1e-10
+    with pytest.raises(_lib.EfeaError, match="not converged"):
+        dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond=precond, maxit=32).run()
+
+
 @pytest.mark.parametrize("dof_n,precond", [(1, "bj"), (2, "two-level")])
 def test_zero_and_non_finite_right_hand_sides(dof_n, precond):
     A, b, x0, known = _system(Q(1, 1, 40, 40), dof_n)
