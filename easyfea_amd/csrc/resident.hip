@@ -44,8 +44,8 @@
 // iteration.  The waits need all blocks on the chip at once: a plan has at
 // most one block per CU, kernels of other streams only delay the blocks they
 // keep out, and the resident solves of a process are queued one after the
-// other (each waits for the event of the last one if that ran on another
-// stream), so that two of them never hold half of the chip each.
+// other (each waits for the event of the last one), so that two of them never
+// hold half of the chip each.
 // (hipLaunchCooperativeKernel gives the same by sending the launch through
 // the runtime's transfer queue: 110 to 140 us more per solve in a program that
 // had used several streams.)
@@ -1081,15 +1081,11 @@ static int res_launch(const ResidentPlan& P, const ResArgs& A, const ResWork& W,
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// The last resident solve queued on each device: its stream and the event
-// recorded behind it (events live as long as the process).
-struct ResLast {
-  hipStream_t stream;
-  hipEvent_t done;
-};
+// The event recorded behind the last resident solve queued on each device
+// (events live as long as the process).
 constexpr int RES_DEVICES = 64;
 static std::mutex res_mutex;
-static ResLast res_last[RES_DEVICES];
+static hipEvent_t res_last[RES_DEVICES];
 
 // This thread's event of poll slot `slot` on device dev (null: creation failed).
 static hipEvent_t res_event(int dev, int slot) {
@@ -1152,8 +1148,10 @@ int solve_resident(const ResidentPlan& P, int Nnode, const int* node_ptr, const 
     A.resume = resume;
     const unsigned nb = (unsigned)((nwords + 1023) / 1024 < 1024 ? (nwords + 1023) / 1024 : 1024);
     std::lock_guard<std::mutex> lock(res_mutex);
-    ResLast& last = res_last[dev];
-    if (last.done && last.stream != s && hipStreamWaitEvent(s, last.done, 0) != hipSuccess) {
+    // also on what looks like the last solve's stream: a handle may name another
+    // stream by now, or one for each thread (hipStreamPerThread)
+    hipEvent_t& last = res_last[dev];
+    if (last && hipStreamWaitEvent(s, last, 0) != hipSuccess) {
       set_error("resident: the last solve's event could not be waited for");
       return EFEA_ERR_HIP;
     }
@@ -1177,8 +1175,7 @@ int solve_resident(const ResidentPlan& P, int Nnode, const int* node_ptr, const 
       set_error("resident: event not recorded");
       return EFEA_ERR_HIP;
     }
-    last.stream = s;
-    last.done = done;
+    last = done;
     return 0;
   };
   auto refused = [&](int rc) {

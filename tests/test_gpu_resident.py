@@ -260,6 +260,41 @@ def test_two_threads_on_their_own_streams():
             assert resident and torch.equal(x, want[k])
 
 
+def test_streams_of_one_handle():
+    """hipStreamPerThread names another stream in each thread: the solves of two
+    threads on it still take the chip in turn."""
+    import threading
+
+    per_thread = 2
+    jobs, want, failed = [], [], []
+    for k in range(2):
+        A, b, x0, known = _system(T(1, 1, 251, 240 + 3 * k), 2, seed=k)
+        want.append(_run(A, b, x0, known, "two-level", "auto")[0].x)
+        job = dv.SolveJob(A, b, x0.clone(), known, "fp64", 1e-12, 1e-10, precond="two-level")
+        job._prepare()
+        assert job.resident.plan.nblk > 128  # two do not fit the chip together
+        jobs.append((job, x0, dv.Workspace()))
+
+    def work(k):
+        job, x0, ws = jobs[k]
+        raw = (C.c_double * 4)()
+        for _ in range(6):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                job.x.copy_(x0)
+                torch.cuda.current_stream().synchronize()
+            if _lib.call("efea_solve_resident", *job._resident_args(ws, 0), per_thread, raw) or raw[3] != 1 \
+                    or not torch.equal(job.x, want[k]):
+                failed.append(k)
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+
+
 @pytest.mark.parametrize("precond", ["bj", "two-level"])
 def test_a_grid_cap_keeps_the_launch_per_step_iteration(precond):
     A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
