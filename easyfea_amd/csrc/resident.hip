@@ -63,6 +63,7 @@
 // (Simulations/Solvers.py:502-553) with _Solve_Axb's backends
 // (Solvers.py:225-394).
 #include <mutex>
+#include <vector>
 
 #include "coarse_device.h"
 #include "resident.h"
@@ -1081,17 +1082,38 @@ static int res_launch(const ResidentPlan& P, const ResArgs& A, const ResWork& W,
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// The event recorded behind the last resident solve queued on each device
-// (events live as long as the process).
 constexpr int RES_DEVICES = 64;
 static std::mutex res_mutex;
+// The event recorded behind the last resident solve queued on each device.
 static hipEvent_t res_last[RES_DEVICES];
+// Events of threads that have ended, for the next ones (never destroyed:
+// res_last may still name one; leaked, so that they outlive every thread).
+static std::vector<hipEvent_t>* const res_free = new std::vector<hipEvent_t>[RES_DEVICES];
+
+struct ResEvents {
+  hipEvent_t ev[RES_DEVICES][2] = {};
+  ~ResEvents() {
+    std::lock_guard<std::mutex> lock(res_mutex);
+    for (int d = 0; d < RES_DEVICES; ++d)
+      for (hipEvent_t e : ev[d])
+        if (e) res_free[d].push_back(e);
+  }
+};
 
 // This thread's event of poll slot `slot` on device dev (null: creation failed).
 static hipEvent_t res_event(int dev, int slot) {
-  static thread_local hipEvent_t ev[RES_DEVICES][2];
-  hipEvent_t& e = ev[dev][slot];
-  if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+  static thread_local ResEvents own;
+  hipEvent_t& e = own.ev[dev][slot];
+  if (e) return e;
+  {
+    std::lock_guard<std::mutex> lock(res_mutex);
+    if (!res_free[dev].empty()) {
+      e = res_free[dev].back();
+      res_free[dev].pop_back();
+      return e;
+    }
+  }
+  if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
     (void)hipGetLastError();
     e = nullptr;
   }

@@ -260,6 +260,28 @@ def test_two_threads_on_their_own_streams():
             assert resident and torch.equal(x, want[k])
 
 
+def test_a_thread_for_each_solve():
+    """Short-lived threads (each takes its event over from one that has ended)."""
+    import threading
+
+    A, b, x0, known = _system(Q(1, 1, 60, 60), 2)
+    want = _run(A, b, x0, known, "two-level", "auto")[0].x
+    got = []
+
+    def work():
+        with torch.cuda.stream(streams[len(got) % 2]):
+            job, info = _run(A, b, x0, known, "two-level", "auto")
+            got.append(info.resident and not info.fallback and torch.equal(job.x, want))
+
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(12):
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+    assert got == [True] * 12
+
+
 def test_streams_of_one_handle():
     """hipStreamPerThread names another stream in each thread: the solves of two
     threads on it still take the chip in turn."""
