@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes as C
 import threading
 import time
+import weakref
 from dataclasses import dataclass
 from typing import Callable, Optional
 
@@ -963,6 +964,7 @@ class SolveJob:
         else:
             entry, args = kind, (self._pcgp_args if kind == "pcgp" else self._pcg2p_args)(ws, check_every, budget)
         s = stream_ptr()
+        PendingSolve.end_open()
         _lib.call(f"efea_{entry}_start", *args, s)
         return PendingSolve(self, ws, kind, args, s, entry)
 
@@ -1048,22 +1050,60 @@ class PendingSolve:
     continues it if the queued iterations were not enough.  ``resumed`` is
     then True: the solution changed after the queued iterations (further
     iterations, or a fallback solve), and work queued from it in between must
-    be redone."""
+    be redone.  A thread's read-back buffer holds one start at a time: the next
+    start ends one that is still open (a simulation whose load step raised),
+    and ``finish`` returns what that gave.  Finished on another thread, whose
+    buffer holds nothing of it, the solve is done again."""
+
+    _of_thread = threading.local()  # .last: the thread's last start, while its owner keeps it
 
     def __init__(self, job: SolveJob, ws: Workspace, kind: str, args: tuple, stream: int, entry: str):
         self.job, self.ws, self.kind, self.args, self.stream = job, ws, kind, args, stream
         self.entry = entry  # of the C functions: kind's pipelined solve, or "resident"
         self.resumed = False
+        self._ended: Optional[SolveInfo] = None
+        self._error: Optional[_lib.EfeaError] = None
+        PendingSolve._of_thread.last = weakref.ref(self)
+
+    @classmethod
+    def _open(cls) -> Optional["PendingSolve"]:
+        """This thread's last start, if it has not been finished."""
+        p = getattr(cls._of_thread, "last", lambda: None)()
+        return p if p is not None and p._ended is None and p._error is None else None
+
+    @classmethod
+    def end_open(cls) -> None:
+        p = cls._open()
+        if p is not None:
+            try:
+                p.finish()
+            except _lib.EfeaError:
+                pass  # its own finish raises it
 
     def finish(self, raise_on_fail: bool = True) -> SolveInfo:
         job = self.job
+        if self._error is not None:
+            raise self._error
+        if self._ended is not None:
+            return self._ended
         raw = (C.c_double * 4)()
         resumed = C.c_int(0)
-        rc = _lib.call(f"efea_{self.entry}_finish", *self.args, self.stream, C.cast(raw, C.c_void_p),
-                       C.byref(resumed))
-        si = job._conclude(self.ws, rc, job.info(raw), raise_on_fail)
+        if PendingSolve._open() is self:
+            rc = _lib.call(f"efea_{self.entry}_finish", *self.args, self.stream, C.cast(raw, C.c_void_p),
+                           C.byref(resumed))
+            si = job.info(raw)
+        else:
+            torch.cuda.synchronize()  # the start, on whichever stream
+            job.x.copy_(job.x0)
+            rc, si = job._solve_once(self.ws)
+            resumed.value = 1
         self.resumed = bool(resumed.value) or rc != 0
-        return si
+        try:
+            self._ended = job._conclude(self.ws, rc, si, raise_on_fail)
+        except _lib.EfeaError as e:
+            self._error = e
+            raise
+        return self._ended
 
 
 def solve(A: DeviceCsr, b: torch.Tensor, x: torch.Tensor, known: Optional[torch.Tensor], mode: str,

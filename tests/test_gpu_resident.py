@@ -260,6 +260,43 @@ def test_two_threads_on_their_own_streams():
             assert resident and torch.equal(x, want[k])
 
 
+@pytest.mark.parametrize("mode,entry", [("fp64", "resident"), ("mixed", "pcgp")])
+def test_a_start_ends_its_thread_s_open_one(mode, entry, monkeypatch):
+    """A solve left open with too few iterations queued, as by a load step that
+    raised, then another one's start on the same thread: both end as whole
+    solves do, and so does one finished by another thread."""
+    import threading
+
+    monkeypatch.setattr(dv, "MIXED_MIN_MATRIX_BYTES", 0)
+    systems = [_system(Q(1, 1, 40 + k, 33), 1, seed=k) for k in range(2)]
+
+    def job(k, expected):
+        A, b, x0, known = systems[k]
+        return dv.SolveJob(A, b, x0.clone(), known, mode, 1e-12, 1e-10, precond="bj", expected_iterations=expected)
+
+    whole = [job(k, 60) for k in range(2)]
+    want = [w.run() for w in whole]
+
+    def check(k, j, info):
+        assert info.status == 1 and not info.fallback and info.iterations == want[k].iterations > 20
+        assert torch.equal(j.x, whole[k].x)
+
+    jobs = [job(0, 3), job(1, 60)]
+    first, second = [j.start() for j in jobs]
+    assert first.entry == second.entry == entry
+    for p in (second, first):
+        check(jobs.index(p.job), p.job, p.finish())
+    assert first.resumed and first.finish() is first.finish()
+
+    j = job(0, 60)
+    pending = j.start()
+    t = threading.Thread(target=pending.finish)
+    t.start()
+    t.join()
+    assert pending.resumed
+    check(0, j, pending.finish())
+
+
 def test_a_thread_for_each_solve():
     """Short-lived threads (each takes its event over from one that has ended)."""
     import threading
