@@ -33,6 +33,7 @@ class CsrMap:
     seg_ptr: np.ndarray  # int32 (nnz+1,)
     perm: np.ndarray  # int32 (Ne*nd*nd,)
     max_neighbours: int
+    repeated: bool  # an element names a node twice
 
     @property
     def nnz(self) -> int:
@@ -146,6 +147,8 @@ def build_csr_map(connect: np.ndarray, Nn: int, dof_n: int) -> CsrMap:
         seg_ptr=seg_ptr.astype(np.int32),
         perm=perm.astype(np.int32),
         max_neighbours=int(cnt.max()) if cnt.size else 0,
+        # each (element, node) adds one pair to the node's own slot, a node named twice four
+        repeated=int(cntp[node_cols == row_node].sum()) != Ne * nPe,
     )
 
 

@@ -57,8 +57,8 @@ __global__ void __launch_bounds__(256) k_row_counts(int Nn, int dn, const int* _
   counts[n + 1] = node_ptr[n + 1] > node_ptr[n] ? seg[s + 1] - seg[s] : 0;
 }
 
-// A wave per node, a lane per (incidence, element node).  repeated: set where an
-// element names a node twice.
+// A wave per node, a lane per (incidence, element node).  repeated (may be null):
+// set where an element names a node twice.
 __global__ void __launch_bounds__(64) k_row_plan(int dn, int nPe, const int* __restrict__ node_ptr,
                                                  const int* __restrict__ node_cols, const int* __restrict__ seg,
                                                  const int* __restrict__ perm, const int* __restrict__ connect,
@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(64) k_row_plan(int dn, int nPe, const int* __r
     const int e = entry / (nd * nd), li = entry % (nd * nd) / nd / dn;
     if (lj == 0) {
       inc[i0 + k] = e * 16 + li;
-      if (entry % nd / dn != li) *repeated = 1;
+      if (repeated && entry % nd / dn != li) *repeated = 1;
     }
     pos[(int64_t)(i0 + k) * nPe + lj] = (unsigned short)place(node_cols, p0, p1, connect[(int64_t)e * nPe + lj]);
   }

@@ -210,7 +210,7 @@ int efea_row_plan(int Nn, int dof_n, int nPe, const int32_t* node_ptr, const int
                   const int32_t* seg_ptr, const int32_t* perm, const int32_t* connect, const int32_t* inc_ptr,
                   int32_t* inc, uint16_t* pos, int32_t* repeated, void* stream) {
   if (Nn <= 0 || dof_n < 1 || nPe < 1 || nPe > 16 || !node_ptr || !node_cols || !seg_ptr || !perm || !connect ||
-      !inc_ptr || !inc || !pos || !repeated) {
+      !inc_ptr || !inc || !pos) {
     set_error("efea_row_plan: null pointer, empty mesh or more than 16 nodes per element");
     return EFEA_ERR_ARG;
   }

@@ -154,23 +154,20 @@ class DeviceMesh:
         if "row_incidence" not in d:
             p = self.pattern(dof_n)
             fits = p.host.max_neighbours <= _lib.load().efea_assemble_max_neighbours(self.code) and self.Ne < 1 << 27
-            d["row_incidence"] = self._row_incidence(p) if fits else None
+            d["row_incidence"] = self._row_incidence(p) if fits and not p.host.repeated else None
         return d["row_incidence"]
 
-    def _row_incidence(self, p: "CsrPattern") -> Optional[tuple]:
+    def _row_incidence(self, p: "CsrPattern") -> tuple:
         counts = torch.empty(self.Nn + 1, dtype=torch.int32, device="cuda")
         inc = torch.empty(self.Ne * self.nPe, dtype=torch.int32, device="cuda")
         pos = torch.empty((self.Ne * self.nPe, self.nPe), dtype=torch.int16, device="cuda")
-        repeated = torch.zeros(1, dtype=torch.int32, device="cuda")
         _lib.call("efea_row_counts", self.Nn, p.dof_n, ptr(p.node_ptr), ptr(p.node_cols), ptr(p.seg), ptr(counts),
                   stream_ptr())
         inc_ptr = counts.cumsum(0, dtype=torch.int32)
-        # a repeated node gives its node more incidences than the lists hold
-        if int(inc_ptr[-1]) != inc.numel():
-            return None
         _lib.call("efea_row_plan", self.Nn, p.dof_n, self.nPe, ptr(p.node_ptr), ptr(p.node_cols), ptr(p.seg),
-                  ptr(p.perm), ptr(self.connect), ptr(inc_ptr), ptr(inc), ptr(pos), ptr(repeated), stream_ptr())
-        return None if int(repeated) else (inc_ptr, inc, pos)  # the copy to the host waits: any stream may use them
+                  ptr(p.perm), ptr(self.connect), ptr(inc_ptr), ptr(inc), ptr(pos), None, stream_ptr())
+        torch.cuda.current_stream().synchronize()  # kept with the mesh: any stream may use them
+        return inc_ptr, inc, pos
 
     def node_values(self, values_e: torch.Tensor) -> torch.Tensor:
         """Element values (Ne, k) -> node values (Nn, k) (``Mesh.Get_Node_Values``)."""

@@ -81,8 +81,9 @@ int efea_assemble_max_neighbours(int elem_type);
 /* Its plan from the scatter map (seg_ptr, perm of efea_csr_scatter).
  * efea_row_counts: counts (Nn + 1) = 0, then each node's incidences; their
  * running sum is inc_ptr.  efea_row_plan fills inc and pos (rows of fewer than
- * 65536 nodes) and sets *repeated (zeroed by the caller) where an element names
- * a node twice, which efea_elastic_assemble does not take. */
+ * 65536 nodes) and sets *repeated (zeroed by the caller; may be null) where an
+ * element names a node twice, which efea_elastic_assemble does not take; inc and
+ * pos must then hold the running sum's last value, more than the elements' nodes. */
 int efea_row_counts(int Nn, int dof_n, const int32_t* node_ptr, const int32_t* node_cols, const int32_t* seg_ptr,
                     int32_t* counts, void* stream);
 int efea_row_plan(int Nn, int dof_n, int nPe, const int32_t* node_ptr, const int32_t* node_cols,

@@ -126,6 +126,16 @@ def test_row_incidence_lists_each_pair_once(et, dof_n):
         assert np.array_equal(row[pos[rows]], mesh.connect[e])
 
 
+@pytest.mark.parametrize("dof_n", [1, 2])
+def test_the_map_tells_a_repeated_node(dof_n):
+    con = ea.quad4_rectangle(3.0, 2.0, 4, 3).connect
+    assert not build_csr_map(con, 21, dof_n).repeated  # (and a node of no element)
+    for k in range(3):
+        twice = con.copy()
+        twice[7, 3] = twice[7, k]
+        assert build_csr_map(twice, 21, dof_n).repeated
+
+
 @pytest.mark.gpu
 def test_a_repeated_node_keeps_element_matrices():
     """A QUAD4 mesh whose last element is collapsed to a triangle."""
