@@ -113,6 +113,8 @@ SIGNATURES = {
          vp, sz, f64, f64, i32, i32, i32, vp, vp, vp],
     ),
     "efea_resident_shape": (i32, [i32, i32, i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
+    "efea_resident_bisect": (i32, [i32, vp, i32, vp, vp]),
+    "efea_resident_neighbours": (i32, [i32, vp, vp, i32, i32, i32, i32, vp, vp, vp, vp, i32, vp, vp, vp, vp, vp, vp]),
     "efea_resident_fits": (i32, [_plan]),
     "efea_resident_workspace_bytes": (sz, [i32, _plan]),
     "efea_solve_resident": (i32, _resident + [vp]),

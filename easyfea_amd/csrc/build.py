@@ -9,7 +9,7 @@ PKG = os.path.dirname(HERE)
 ROOT = os.path.dirname(PKG)
 SOURCES = ["capi.hip", "elements.hip", "sparse.hip", "batch.hip", "coarse.hip", "phasefield.hip", "postproc.hip",
            "dynamics.hip", "bounded.hip", "pcg2p.hip", "elements_mfma.hip", "pcgp.hip",
-           "bicgstab.hip", "resident.hip", "assemble.hip"]
+           "bicgstab.hip", "resident.hip", "resident_plan.cpp", "assemble.hip"]
 # The phase-field split branches on exact equality of eigenvalues (as the
 # reference does); contracting a*b - c*d into an FMA changes which states
 # compare equal, so that file is compiled operation by operation.
@@ -34,7 +34,7 @@ def build(verbose: bool = False) -> str:
     objs, procs = [], []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
     for src in SOURCES:
-        obj = os.path.join(HERE, "_build", src.replace(".hip", ".o"))
+        obj = os.path.join(HERE, "_build", os.path.splitext(src)[0] + ".o")
         cmd = [HIPCC, *COMPILE_FLAGS, *EXTRA.get(src, []), "-c", "-x", "hip", os.path.join(HERE, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

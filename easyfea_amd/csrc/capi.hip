@@ -628,6 +628,32 @@ int efea_resident_shape(int dof_n, int max_neighbours, int min_passes, int* lane
   return resident_shape(dof_n, max_neighbours, min_passes, lanes, slots, passes);
 }
 
+int efea_resident_bisect(int Nn, const double* coord, int parts, int32_t* order, int32_t* part_ptr) {
+  if (Nn < 1 || parts < 1 || !coord || !order || !part_ptr) {
+    set_error("efea_resident_bisect: null pointer, no nodes or no parts");
+    return EFEA_ERR_ARG;
+  }
+  return resident_bisect(Nn, coord, parts, order, part_ptr);
+}
+
+int efea_resident_neighbours(int Nn, const int32_t* node_ptr, const int32_t* node_cols, int lanes, int slots,
+                             int passes, int nblk, const int32_t* rows, uint16_t* lidx, int32_t* halo_ptr,
+                             int32_t* halo_ex, int halo_room, int32_t* pub, int32_t* pub_ptr, int32_t* pub_pos,
+                             int32_t* self, int32_t* nex, int32_t* max_halo) {
+  if (Nn < 1 || !node_ptr || !node_cols || !rows || !lidx || !halo_ptr || !halo_ex || !pub || !pub_ptr || !pub_pos ||
+      !self || !nex || !max_halo || halo_room < 0) {
+    set_error("efea_resident_neighbours: null pointer or empty system");
+    return EFEA_ERR_ARG;
+  }
+  if ((lanes != 1 && lanes != 2 && lanes != 4) || slots < (lanes == 1 ? 2 : 1) || passes < 1 || nblk < 1 ||
+      (int64_t)nblk * passes * (512 / lanes) > INT32_MAX) {
+    set_error("efea_resident_neighbours: %d lanes, %d slots, %d passes, %d blocks", lanes, slots, passes, nblk);
+    return EFEA_ERR_ARG;
+  }
+  return resident_neighbours(Nn, node_ptr, node_cols, lanes, slots, passes, nblk, rows, lidx, halo_ptr, halo_ex,
+                             halo_room, pub, pub_ptr, pub_pos, self, nex, max_halo);
+}
+
 int efea_resident_fits(const efea_resident_plan* plan) { return plan ? resident_fits(*plan) : 0; }
 
 size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan) {

@@ -34,19 +34,10 @@ def shape(dof_n: int, max_neighbours: int, min_passes: int) -> Optional[tuple]:
 def bisect(coord: np.ndarray, parts: int) -> list:
     """The nodes in ``parts`` compact groups of nearly equal size (recursive
     coordinate bisection), each in increasing order."""
-    out, stack = [], [(np.arange(coord.shape[0]), parts)]
-    while stack:
-        ids, k = stack.pop()
-        if k == 1:
-            out.append(np.sort(ids))
-            continue
-        c = coord[ids]
-        x = c[:, int(np.argmax(c.max(0) - c.min(0)))]
-        h = ids.size * (k // 2) // k
-        order = np.argpartition(x, h) if 0 < h < ids.size else np.arange(ids.size)
-        stack.append((ids[order[h:]], k - k // 2))
-        stack.append((ids[order[:h]], k // 2))
-    return out
+    c = np.ascontiguousarray(coord, dtype=np.float64)
+    order, ptr_ = np.empty(c.shape[0], dtype=np.int32), np.empty(parts + 1, dtype=np.int32)
+    _lib.call("efea_resident_bisect", c.shape[0], c.ctypes.data, parts, order.ctypes.data, ptr_.ctypes.data)
+    return np.split(order, ptr_[1:-1])
 
 
 def block_count(least: int, per_block: int, max_blocks: int, agg: np.ndarray, nc: int) -> int:
@@ -158,52 +149,22 @@ def collection(nm: int, nagg: int, pc: dict) -> np.ndarray:
 def neighbours(rows: torch.Tensor, node_ptr: torch.Tensor, node_cols: torch.Tensor, lanes: int, slots: int,
                passes: int) -> dict:
     """Halo lists, exchange numbers and the local neighbour positions of a
-    layout, as ``include/efea.h`` describes them (torch, on the inputs' device)."""
-    dev = rows.device
+    layout, as ``include/efea.h`` describes them (host tensors)."""
     nblk, nloc = rows.shape
-    Nn = node_ptr.numel() - 1
-    flat = rows.reshape(-1).long()
-    have = torch.nonzero(flat >= 0).flatten()
-    pos = torch.empty(Nn, dtype=torch.int64, device=dev)
-    pos[flat[have]] = have
-    cnt = (node_ptr[1:] - node_ptr[:-1]).long()
-    row = torch.repeat_interleave(torch.arange(Nn, device=dev), cnt)
-    k = torch.arange(row.numel(), device=dev) - node_ptr.long()[row]
-    prow, pcol = pos[row], pos[node_cols.long()]
-    brow = prow // nloc
-    cross = brow != pcol // nloc
-    key = torch.unique(brow[cross] * (nblk * nloc) + pcol[cross])  # by block, then the owner's position
-    hblk, hpos = key // (nblk * nloc), key % (nblk * nloc)
-    halo_ptr = torch.searchsorted(hblk, torch.arange(nblk + 1, device=dev))
-    ex_pos = torch.unique(hpos)
-    pub = torch.full((nblk * nloc,), -1, dtype=torch.int32, device=dev)
-    pub[ex_pos] = torch.arange(ex_pos.numel(), dtype=torch.int32, device=dev)
-    local = pcol % nloc
-    place = torch.searchsorted(key, brow[cross] * (nblk * nloc) + pcol[cross])
-    local[cross] = nloc + place - halo_ptr[brow[cross]]
-    if lanes == 1:  # scalar rows: the node itself first, without an entry
-        own = node_cols.long() == row
-        self_k = torch.zeros(Nn, dtype=k.dtype, device=dev)  # a node of no element has an empty row
-        self_k[row[own]] = k[own]
-        k = torch.where(own, 0, torch.where(k < self_k[row], k + 1, k))
-    per = 64 // lanes
-    p = prow % nloc
-    chunk = p // per
-    thread = (chunk % WAVES) * 64 + (p % per) * lanes + k % lanes
-    slot, kept = k // lanes, slots
-    self_pos = torch.zeros(nblk * nloc, dtype=torch.int32, device=dev)
-    if lanes == 1:
-        slot, kept = slot - 1, slots - 1
-        self_pos[pos] = self_k.int()
-    at = ((brow * passes + chunk // WAVES) * kept + slot) * (64 * WAVES) + thread
-    lidx = torch.zeros(nblk * passes * kept * 64 * WAVES, dtype=torch.int16, device=dev)
-    if lanes == 1:
-        at, local = at[~own], local[~own]
-    lidx[at] = local.to(torch.int16)
-    pub_ptr = torch.searchsorted(ex_pos, torch.arange(nblk + 1, device=dev) * nloc)
-    return dict(lidx=lidx, halo_ptr=halo_ptr.int(), halo_ex=pub[hpos].contiguous(), pub=pub,
-                pub_ptr=pub_ptr.int(), pub_pos=(ex_pos % nloc).int(), self=self_pos,
-                nex=int(ex_pos.numel()), max_halo=int((halo_ptr[1:] - halo_ptr[:-1]).max()))
+    kept = slots - 1 if lanes == 1 else slots  # a scalar row's own node has no entry
+    rows, node_ptr, node_cols = (t.to(torch.int32).contiguous() for t in (rows, node_ptr, node_cols))
+    i32 = dict(dtype=torch.int32)
+    out = dict(lidx=torch.empty(nblk * passes * kept * 64 * WAVES, dtype=torch.int16),
+               halo_ptr=torch.empty(nblk + 1, **i32), halo_ex=torch.empty(node_cols.numel(), **i32),
+               pub=torch.empty(nblk * nloc, **i32), pub_ptr=torch.empty(nblk + 1, **i32),
+               pub_pos=torch.empty(nblk * nloc, **i32), self=torch.empty(nblk * nloc, **i32))
+    nex, max_halo = C.c_int(), C.c_int()
+    _lib.call("efea_resident_neighbours", node_ptr.numel() - 1, node_ptr.data_ptr(), node_cols.data_ptr(), lanes,
+              slots, passes, nblk, rows.data_ptr(), out["lidx"].data_ptr(), out["halo_ptr"].data_ptr(),
+              out["halo_ex"].data_ptr(), out["halo_ex"].numel(), *[out[n].data_ptr() for n in (
+                  "pub", "pub_ptr", "pub_pos", "self")], C.addressof(nex), C.addressof(max_halo))
+    return dict(out, halo_ex=out["halo_ex"][:int(out["halo_ptr"][-1])], pub_pos=out["pub_pos"][:nex.value],
+                nex=nex.value, max_halo=max_halo.value)
 
 
 class Resident:
@@ -226,10 +187,12 @@ class Resident:
         lanes, slots, passes, rows, chunk_agg = lay
         if rows.shape[1] + pattern.Nn > 2**31 - 1:
             return None
+        h = pattern.host
+        nb = neighbours(torch.from_numpy(rows), torch.from_numpy(h.node_ptr), torch.from_numpy(h.node_cols), lanes,
+                        slots, passes)
         rows_dev = torch.from_numpy(rows).to("cuda")
-        nb = neighbours(rows_dev, pattern.node_ptr, pattern.node_cols, lanes, slots, passes)
-        keep = dict(rows=rows_dev, **{n: nb[n] for n in ("lidx", "halo_ptr", "halo_ex", "pub", "pub_ptr",
-                                                            "pub_pos", "self")})
+        keep = dict(rows=rows_dev, **{n: nb[n].to("cuda") for n in ("lidx", "halo_ptr", "halo_ex", "pub", "pub_ptr",
+                                                                    "pub_pos", "self")})
         pl = _lib.ResidentPlan(dof_n=pattern.dof_n, slots=slots, passes=passes, nblk=rows.shape[0],
                                max_halo=nb["max_halo"], nex=nb["nex"])
         if rows.shape[1] + nb["max_halo"] > 65535:

@@ -448,6 +448,20 @@ typedef struct efea_resident_plan {
  * included) with at least min_passes passes: returns 1 and its lanes per node,
  * slots per lane and passes, or 0 when there is none. */
 int efea_resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, int* slots, int* passes);
+/* The parts of a plan that follow from the pattern alone, on host arrays.
+ * efea_resident_bisect: the nodes in `parts` compact groups of nearly equal size
+ * (recursive bisection along the longest side of their coordinates, coord 3 per
+ * node): order (Nn) lists them by group, increasing within one, part_ptr
+ * (parts + 1) the groups.  efea_resident_neighbours fills lidx, halo_ptr,
+ * halo_ex (at most halo_room entries; node_ptr[Nn] always suffice), pub,
+ * pub_ptr, pub_pos (nblk * nloc), self (also zeroed for dof_n > 1), nex and
+ * max_halo from rows, which must name every node once; lanes and slots as
+ * efea_resident_shape gives them. */
+int efea_resident_bisect(int Nn, const double* coord, int parts, int32_t* order, int32_t* part_ptr);
+int efea_resident_neighbours(int Nn, const int32_t* node_ptr, const int32_t* node_cols, int lanes, int slots,
+                             int passes, int nblk, const int32_t* rows, uint16_t* lidx, int32_t* halo_ptr,
+                             int32_t* halo_ex, int halo_room, int32_t* pub, int32_t* pub_ptr, int32_t* pub_pos,
+                             int32_t* self, int32_t* nex, int32_t* max_halo);
 /* 1 if a block of the plan (sizes only; the pointers are not read) fits a CU's LDS. */
 int efea_resident_fits(const efea_resident_plan* plan);
 size_t efea_resident_workspace_bytes(int Nnode, const efea_resident_plan* plan);

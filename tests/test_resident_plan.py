@@ -8,6 +8,7 @@ import torch
 
 import easyfea_amd as ea
 from easyfea_amd import resident as R
+from easyfea_amd._lib import EfeaError
 from easyfea_amd.assembly_map import build_csr_map
 from easyfea_amd.coarse import aggregate
 from easyfea_amd.mesh import tetra4_box
@@ -117,6 +118,31 @@ def _check_collection(table, nblk, nm, pc):
             for m in range(nm):
                 want.setdefault(pc["piece_agg"][j] * nm + m, []).append(k * line + 3 + i * nm + m)
     assert got == want
+
+
+@pytest.mark.parametrize("n,parts", [(1, 1), (7, 3), (5000, 17), (300_000, 256)])  # the last one by several threads
+def test_bisection_parts(n, parts):
+    rng = np.random.default_rng(n)
+    coord = np.zeros((n, 3))
+    coord[:, :2] = rng.integers(0, 600, (n, 2))  # many equal coordinates
+    coord[rng.integers(0, n, 3), 2] = [0.0, np.inf, np.nan]
+    out = R.bisect(coord, parts)
+    assert len(out) == parts and np.array_equal(np.sort(np.concatenate(out)), np.arange(n))
+    assert all((np.diff(p) > 0).all() and p.size <= -(-n // parts) for p in out)
+    again = R.bisect(coord, parts)
+    assert all(np.array_equal(a, b) for a, b in zip(out, again))
+
+
+def test_neighbours_refuses_rows_that_do_not_fit():
+    mesh, m, _, (lanes, slots, passes, rows, _) = _plan("quad 33x17", 1, None, 256)
+    graph = torch.from_numpy(m.node_ptr), torch.from_numpy(m.node_cols)
+    for bad in (np.where(rows == 5, -1, rows), np.where(rows == 5, mesh.Nn, rows)):  # a node without a place, none
+        with pytest.raises(EfeaError, match="position"):
+            R.neighbours(torch.from_numpy(bad), *graph, lanes, slots, passes)
+    with pytest.raises(EfeaError, match="slots"):
+        R.neighbours(torch.from_numpy(rows), *graph, lanes, slots - 2, passes)
+    with pytest.raises(EfeaError, match="lanes"):
+        R.neighbours(torch.from_numpy(rows), *graph, 3, slots, passes)
 
 
 def test_layout_refuses_what_no_variant_holds():
