@@ -14,15 +14,13 @@ vp = C.c_void_p
 i32, i64, f64, sz = C.c_int, C.c_int64, C.c_double, C.c_size_t
 
 
-
 class ResidentPlan(C.Structure):
     """``efea_resident_plan`` of ``include/efea.h``."""
 
     _fields_ = ([(n, C.c_int32) for n in ("dof_n", "slots", "passes", "nblk", "max_halo", "nex", "nagg", "npiece",
                                           "max_pieces", "ncollect")]
                 + [(n, vp) for n in ("rows", "lidx", "halo_ptr", "halo_ex", "pub", "pub_ptr", "pub_pos", "self",
-                                     "piece_ptr", "piece_agg", "piece_chunk",
-                                     "chunk_piece", "collect")])
+                                     "piece_ptr", "piece_agg", "chunk_piece", "collect")])
 
 
 _plan = C.POINTER(ResidentPlan)

@@ -675,7 +675,7 @@ static int resident_check(const char* fn, const efea_resident_plan* P, int Nnode
     return EFEA_ERR_ARG;
   }
   if (P->nagg > 0 && (P->dof_n < 2 || P->npiece <= 0 || P->max_pieces <= 0 || !P->piece_ptr || !P->piece_agg ||
-                      !P->piece_chunk || !P->chunk_piece || !P->collect || !rel || !Ainv ||
+                      !P->chunk_piece || !P->collect || !rel || !Ainv ||
                       ld < coarse_ld(P->nagg, P->dof_n))) {
     set_error("%s: incomplete coarse space", fn);
     return EFEA_ERR_ARG;

@@ -291,12 +291,12 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
   if (t < RING) ring[t] = 0;
   // the lane's position of pass p
   auto at = [&](int p) { return G == 1 ? p * RT + t : (p * RNW + wv) * NPC + q; };
-  // a uniform address, formed anew each time: the loop's own copies of what is
-  // added to it would fill the registers
   // between passes: several passes' loads in flight would spill
   auto fence = [] {
     if constexpr (NP > 1) __builtin_amdgcn_sched_barrier(0);
   };
+  // a uniform address, formed anew each time: the loop's own copies of what is
+  // added to it would fill the registers
   using Global = __attribute__((address_space(1))) double;
   auto fresh = [](double* a) {
     auto* f = (Global*)a;
@@ -991,9 +991,9 @@ static inline size_t res_xp_bytes(const ResidentPlan& P) {
 
 // BIG's streamed passes.
 static inline size_t res_vs_bytes(const ResidentPlan& P) {
-#define STREAM(D, SV, NPV, ILV)                             \
+#define STREAM(D, SV, NPV, BIG)                             \
   if (P.dof_n == D && P.slots == SV && P.passes == NPV)     \
-    return align256(8 * (size_t)P.nblk * RT * SV * (NPV - ResPasses<SV, NPV, ILV>::KEPT));
+    return align256(8 * (size_t)P.nblk * RT * SV * (NPV - ResPasses<SV, NPV, BIG>::KEPT));
   EFEA_RESIDENT(STREAM)
 #undef STREAM
   return 0;
@@ -1034,7 +1034,7 @@ static ResWork res_carve(void* ws, int Nnode, int dof_n, const ResidentPlan& P, 
 
 int resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, int* slots, int* passes) {
   int best = 0;
-#define SHAPE(D, SV, NPV, ILV)                                                                      \
+#define SHAPE(D, SV, NPV, BIG)                                                                      \
   if (!best && D == dof_n && ResLanes<D>::G * SV >= max_neighbours && NPV >= min_passes) {          \
     best = 1;                                                                                       \
     *lanes = ResLanes<D>::G;                                                                        \
@@ -1049,10 +1049,10 @@ int resident_shape(int dof_n, int max_neighbours, int min_passes, int* lanes, in
 // LDS bytes a block of the plan needs without (rows = 0) or with its rows of
 // the coarse inverse in LDS; 0 when no kernel variant matches.
 static size_t res_lds_bytes(const ResidentPlan& P, int two, int rows) {
-#define LDSB(D, SV, NPV, ILV)                                                             \
+#define LDSB(D, SV, NPV, BIG)                                                             \
   if (P.dof_n == D && P.slots == SV && P.passes == NPV)                                   \
-    return 8 * (size_t)(two ? res_lds<D, true>(P, SV, NPV, ILV, rows != 0).total          \
-                            : res_lds<D, false>(P, SV, NPV, ILV, false).total);
+    return 8 * (size_t)(two ? res_lds<D, true>(P, SV, NPV, BIG, rows != 0).total          \
+                            : res_lds<D, false>(P, SV, NPV, BIG, false).total);
   EFEA_RESIDENT(LDSB)
 #undef LDSB
   return 0;
@@ -1179,13 +1179,13 @@ int solve_resident(const ResidentPlan& P, int Nnode, const int* node_ptr, const 
     }
     hipLaunchKernelGGL(k_res_empty, dim3(nb ? nb : 1), dim3(256), 0, s, nwords, W.hx, pb);
     int rc = 1;
-#define RUN(D, SV, NPV, ILV)                                                                \
+#define RUN(D, SV, NPV, BIG)                                                                \
   if (P.dof_n == D && P.slots == SV && P.passes == NPV) {                                   \
     if constexpr (D == 1)                                                                   \
-      rc = two ? 1 : res_launch<D, SV, NPV, false, ILV>(P, A, W, lds, dev, s);                   \
+      rc = two ? 1 : res_launch<D, SV, NPV, false, BIG>(P, A, W, lds, dev, s);              \
     else                                                                                    \
-      rc = two ? res_launch<D, SV, NPV, true, ILV>(P, A, W, lds, dev, s)                         \
-               : res_launch<D, SV, NPV, false, ILV>(P, A, W, lds, dev, s);                       \
+      rc = two ? res_launch<D, SV, NPV, true, BIG>(P, A, W, lds, dev, s)                    \
+               : res_launch<D, SV, NPV, false, BIG>(P, A, W, lds, dev, s);                  \
   }
     EFEA_RESIDENT(RUN)
 #undef RUN

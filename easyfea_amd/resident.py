@@ -106,7 +106,8 @@ def layout(coord: Optional[np.ndarray], Nn: int, dof_n: int, max_neighbours: int
 
 
 def pieces(chunk_agg: np.ndarray) -> dict:
-    """The runs of one block's chunks of one aggregate, numbered through."""
+    """The runs of one block's chunks of one aggregate, numbered through
+    (``piece_chunk``: each one's first and past-last chunk, for checks of a plan)."""
     nblk, nch = chunk_agg.shape
     new = chunk_agg >= 0
     new[:, 1:] &= chunk_agg[:, 1:] != chunk_agg[:, :-1]
@@ -202,7 +203,7 @@ class Resident:
             pl.nagg, pl.npiece, pl.max_pieces = cs.nagg, pc["piece_agg"].size, pc["max_pieces"]
             pc["collect"] = collection(cs.nm, cs.nagg, pc)
             pl.ncollect = pc["collect"].shape[0]
-            for n in ("piece_ptr", "piece_agg", "piece_chunk", "chunk_piece", "collect"):
+            for n in ("piece_ptr", "piece_agg", "chunk_piece", "collect"):
                 keep[n] = torch.from_numpy(pc[n].astype(np.int32)).to("cuda")
         for n, t in keep.items():
             setattr(pl, n, t.data_ptr() if t.numel() else rows_dev.data_ptr())  # never null

@@ -413,9 +413,8 @@ int efea_pcg2p_finish(int precision, int Nnode, int dof_n, int group, const int3
  *   with aggregates (nagg > 0, else 0 and the pointers null), whose nodes
  *     fill whole chunks in aggregate order: pieces are the runs of one
  *     block's chunks of one aggregate, numbered through; piece_ptr (nblk + 1),
- *     piece_agg (npiece), piece_chunk (2 npiece: first and past-last chunk of
- *     its block), chunk_piece (nblk * 8 * passes: piece of each chunk within its block,
- *     -1 for none); max_pieces: the most pieces of one block;
+ *     piece_agg (npiece), chunk_piece (nblk * 8 * passes: piece of each chunk
+ *     within its block, -1 for none); max_pieces: the most pieces of one block;
  *   collect (ncollect * 256, with aggregates): what thread 256 + c of every
  *     block reads of the restrictions the blocks publish per iteration, entries
  *     collect[i * 256 + c], -1 for none (none after it either): offset |
@@ -440,7 +439,6 @@ typedef struct efea_resident_plan {
   const int32_t* self;
   const int32_t* piece_ptr;
   const int32_t* piece_agg;
-  const int32_t* piece_chunk;
   const int32_t* chunk_piece;
   const int32_t* collect;
 } efea_resident_plan;
