@@ -14,6 +14,7 @@ from easyfea_amd import Models, Simulations, _lib
 from easyfea_amd import device as dv
 from easyfea_amd import resident as R
 from easyfea_amd.mesh import tetra4_box
+from test_resident_plan import irregular
 
 pytestmark = pytest.mark.gpu
 
@@ -77,7 +78,28 @@ CASES = [  # mesh, dof_n, preconditioner, (slots, passes)
     (lambda: tetra4_box(1, 1, 1, 17, 18, 17), 3, "two-level", (4, 1)),
     (lambda: tetra4_box(1, 1, 1, 35, 34, 33), 3, "two-level", (4, 2)),
     (lambda: tetra4_box(1, 1, 1, 6, 5, 4), 3, "bj", (4, 1)),
+    # Delaunay meshes: rows of up to 11 nodes in 2D, 27 in 3D
+    (lambda: irregular(30, 2, 2), 2, "bj", (8, 1)),
+    (lambda: irregular(30, 2, 2), 2, "two-level", (8, 1)),
+    (lambda: irregular(262, 2), 2, "two-level", (8, 2)),
+    (lambda: irregular(30, 2, 2), 1, "bj", (16, 1)),
+    (lambda: irregular(9, 3), 1, "bj", (28, 1)),
+    (lambda: irregular(9, 3), 3, "bj", (7, 1)),
+    (lambda: irregular(17, 3), 3, "two-level", (7, 1)),
+    (lambda: irregular(262, 2), 2, "bj", (8, 2)),
+    (lambda: T(1, 1, 290, 250), 2, "bj", (4, 2)),
+    (lambda: Q(1, 1, 290, 250), 2, "bj", (5, 2)),
+    (lambda: Q(1, 1, 400, 420), 2, "bj", (5, 4)),
+    (lambda: T(1, 1, 400, 420), 2, "two-level", (4, 4)),
+    (lambda: tetra4_box(1, 1, 1, 35, 34, 33), 3, "bj", (4, 2)),
 ]
+
+
+def test_every_variant_has_a_case():
+    """Each of EFEA_RESIDENT, and with aggregates those of two and three DOFs."""
+    shapes = {(d, p, R.shape(d, n, k)[1:]) for d in (1, 2, 3) for n in range(1, 30) for k in range(1, 10)
+              for p in ("bj", "two-level")[:d] if R.shape(d, n, k)}
+    assert shapes == {(d, p, v) for _, d, p, v in CASES}
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))

@@ -5,6 +5,7 @@ published nodes, and the pieces cover each aggregate's chunks."""
 import numpy as np
 import pytest
 import torch
+from scipy.spatial import Delaunay
 
 import easyfea_amd as ea
 from easyfea_amd import resident as R
@@ -23,7 +24,22 @@ def _with_orphans(mesh, at):
     return ea.Mesh({t: new[g.connect] for t, g in mesh.dict_groupElem.items()}, coord)
 
 
+def irregular(n, dim, seed=0):
+    """Delaunay triangles or tetrahedra of an (n + 1)^dim grid whose inner
+    points are moved by up to 0.45 of a cell; flat ones left out."""
+    g = np.stack(np.meshgrid(*[np.arange(n + 1.0)] * dim, indexing="ij"), -1).reshape(-1, dim)
+    move = np.random.default_rng(seed).uniform(-0.45, 0.45, g.shape)
+    g += np.where((g > 0) & (g < n), move, 0.0)
+    con = Delaunay(g).simplices
+    con = con[np.abs(np.linalg.det(g[con[:, 1:]] - g[con[:, :1]])) > 1e-3]
+    coord = np.zeros((len(g), 3))
+    coord[:, :dim] = g / n
+    return ea.Mesh({"TRI3" if dim == 2 else "TETRA4": con}, coord)
+
+
 MESHES = {
+    "irregular 2D": (lambda: irregular(30, 2, 2), 2),
+    "irregular 3D": (lambda: irregular(8, 3), 3),
     # empty rows first, in the middle and last
     "orphans quad 20": (lambda: _with_orphans(ea.quad4_rectangle(1.0, 1.0, 20, 20), [0, 200, 200, 441]), 2),
     "orphan tetra 5": (lambda: _with_orphans(tetra4_box(1.0, 1.0, 1.0, 5, 5, 5), [216]), 3),
