@@ -555,17 +555,19 @@ class ResidentPauses:
         self._row: dict = {}    # device -> solves given up in a row
         self._until: dict = {}  # device -> end of its pause
 
-    def paused(self, device: int) -> bool:
-        return self._until.get(device, 0.0) > self.clock()
+    def paused(self) -> bool:
+        return bool(self._until) and self._until.get(torch.cuda.current_device(), 0.0) > self.clock()
 
-    def gave_up(self, device: int) -> None:
+    def gave_up(self) -> None:
+        device = torch.cuda.current_device()
         with self._lock:
             row = self._row[device] = self._row.get(device, 0) + 1
             if row > 1:
                 self._until[device] = self.clock() + min(self.FIRST * 2.0 ** min(row - 2, 30), self.MOST)
 
-    def succeeded(self, device: int) -> None:
-        if device in self._row:
+    def succeeded(self) -> None:
+        if self._row:
+            device = torch.cuda.current_device()
             with self._lock:
                 self._row.pop(device, None)
                 self._until.pop(device, None)
@@ -725,7 +727,7 @@ class SolveJob:
         not drift), wherever the matrix fits the chip's registers."""
         if self.pipelined_mode is False or self.precision != 64 or self.method != "pcg" or self.max_blocks > 0:
             return None
-        if resident_pauses.paused(torch.cuda.current_device()):
+        if resident_pauses.paused():
             return None
         if self.precond == "two-level":
             return self.A.pattern.resident(self.A.coarse(self.coarse_target))
@@ -904,9 +906,9 @@ class SolveJob:
         isolating = self.isolate is not None and self.A.pattern.coord is not None
         if self.resident is not None:
             if rc == 0:
-                resident_pauses.succeeded(torch.cuda.current_device())
+                resident_pauses.succeeded()
             elif si.replacements:  # as efea_solve_resident reports a wait given up
-                resident_pauses.gave_up(torch.cuda.current_device())
+                resident_pauses.gave_up()
         if rc != 0 and (self.pipelined if self.resident is None else si.status != 0):
             # a pipelined breakdown (rounding in its recurrences) or a resident
             # solve given up: the classic iteration from the same start (not
