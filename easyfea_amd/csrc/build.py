@@ -15,7 +15,12 @@ SOURCES = ["capi.hip", "elements.hip", "sparse.hip", "batch.hip", "coarse.hip", 
 # compare equal, so that file is compiled operation by operation.
 # The time-scheme state update mirrors the reference's numpy expressions
 # operation by operation, which also needs uncontracted arithmetic.
-EXTRA = {"phasefield.hip": ["-ffp-contract=off"], "dynamics.hip": ["-ffp-contract=off"]}
+# The resident solve's waits and sums are short loops in a kernel of 50 KB; where
+# unrelated code moved their starts, an iteration on TRI3 251 x 249 went from 6.67
+# to 6.90 us and back (notched TRI3 200^2 8.10 and 8.27).  On 64-byte lines it is
+# 6.68 (8.06) wherever they land.
+EXTRA = {"phasefield.hip": ["-ffp-contract=off"], "dynamics.hip": ["-ffp-contract=off"],
+         "resident.hip": ["-falign-loops=64"]}
 OUT = os.path.join(PKG, "libefea_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMPILE_FLAGS = [

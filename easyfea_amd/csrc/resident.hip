@@ -178,8 +178,8 @@ template <int DN, int S> struct ResSlots { static constexpr int N = DN == 1 ? S 
 // 64-byte lines of their own (blocks that share a line slow every poll of it:
 // 256 blocks' all-to-all took 8,700 cycles with the scalars of all blocks side
 // by side, 5,800 with a line per block).
-template <int NM>
-__host__ __device__ inline int res_line(const ResidentPlan& P) {
+template <int NM, typename Plan>
+__host__ __device__ inline int res_line(const Plan& P) {
   return (3 + (P.nagg > 0 ? P.max_pieces * NM : 0) + 7) / 8 * 8;
 }
 
@@ -190,8 +190,8 @@ struct ResLds {
   int u, pay, rel, ch, z, zs, rows, item, idx, p, total;
 };
 
-template <int DN, bool TWO>
-__host__ __device__ inline ResLds res_lds(const ResidentPlan& P, int S, int NP, bool BIG, bool cache_rows) {
+template <int DN, bool TWO, typename Plan>
+__host__ __device__ inline ResLds res_lds(const Plan& P, int S, int NP, bool BIG, bool cache_rows) {
   constexpr int NM = Modes<DN>::NM, G = ResLanes<DN>::G;
   const int nloc = RT / G * NP, nc = TWO ? res_columns(P.nagg * NM) : 0;
   ResLds L;
@@ -212,6 +212,27 @@ __host__ __device__ inline ResLds res_lds(const ResidentPlan& P, int S, int NP, 
   L.total = o;
   return L;
 }
+
+// The plan as a kernel argument.  `gap` decides which arguments share a scalar
+// load and so what the compiler keeps in scalar registers.  An iteration of the
+// two-level variants with and without it: QUAD4 32^2 5.24 and 5.40 us, 360 x 39
+// 5.38 and 5.55, TRI3 251 x 249 6.68 and 6.75, HEXA8 31^3 11.86 and 11.91 (30^3
+// 11.73 and 11.52); 8 bytes behind the plan instead: 31^3 12.97.
+struct KernelPlan {
+  int dof_n, slots, passes, nblk, max_halo, nex, nagg, npiece, max_pieces, ncollect;
+  const int* rows;
+  const unsigned short* lidx;
+  const int *halo_ptr, *halo_ex, *pub, *pub_ptr, *pub_pos, *self, *piece_ptr, *piece_agg;
+  const void* gap;
+  const int *chunk_piece, *collect;
+
+  explicit KernelPlan(const ResidentPlan& P)
+      : dof_n(P.dof_n), slots(P.slots), passes(P.passes), nblk(P.nblk), max_halo(P.max_halo), nex(P.nex),
+        nagg(P.nagg), npiece(P.npiece), max_pieces(P.max_pieces), ncollect(P.ncollect), rows(P.rows), lidx(P.lidx),
+        halo_ptr(P.halo_ptr), halo_ex(P.halo_ex), pub(P.pub), pub_ptr(P.pub_ptr), pub_pos(P.pub_pos), self(P.self),
+        piece_ptr(P.piece_ptr), piece_agg(P.piece_agg), gap(nullptr), chunk_piece(P.chunk_piece),
+        collect(P.collect) {}
+};
 
 struct ResWork {
   double *r, *u, *p, *s;   // a paused solve's vectors
@@ -261,7 +282,7 @@ struct ResPasses {
 };
 template <int DN, int S, int NP, bool TWO, bool BIG>
 __global__ void __launch_bounds__(RT, 2)
-k_resident(ResidentPlan P, ResArgs A, ResWork W) {
+k_resident(KernelPlan P, ResArgs A, ResWork W) {
   constexpr int NM = Modes<DN>::NM, G = ResLanes<DN>::G, NPC = 64 / G, NLOC = RT / G * NP;
   constexpr int SN = ResSlots<DN, S>::N, S2 = (SN + 1) / 2, NR = BIG ? 1 : NP;
   constexpr int NV = ResPasses<S, NP, BIG>::KEPT;  // passes whose values stay in registers
@@ -319,7 +340,7 @@ k_resident(ResidentPlan P, ResArgs A, ResWork W) {
     const int p0 = A.node_ptr[n], cnt = A.node_ptr[n + 1] - p0;
     // a node of no element has an empty row: its loads (dropped) go to the first
     // values, where p0 of a last such node would be past the end
-    const int64_t base = cnt > 0 ? (int64_t)DN * DN * p0 : 0;
+    const int64_t base = (int64_t)DN * DN * (cnt > 0 ? p0 : 0);
     const int self = DN == 1 ? P.self[gp] : 0;
     double* vs = W.vs + ((int64_t)blk * (NP - NV) + (p - NV)) * S * RT + t;  // a streamed pass
     bool diag = false, off = false;  // BIG: not zero
@@ -1078,7 +1099,7 @@ static int res_launch(const ResidentPlan& P, const ResArgs& A, const ResWork& W,
     }
     ready = dev;
   }
-  hipLaunchKernelGGL(fn, dim3((unsigned)P.nblk), dim3(RT), lds, s, P, A, W);
+  hipLaunchKernelGGL(fn, dim3((unsigned)P.nblk), dim3(RT), lds, s, KernelPlan(P), A, W);
   return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
