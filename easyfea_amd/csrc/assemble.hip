@@ -18,7 +18,7 @@
 // One wave per block (nothing to synchronise), entries summed in increasing
 // element order (deterministic).  Bound: latency.  The rows (15.5 KB for 8
 // HEXA8 nodes) and the registers (reference gradients held, 250) leave 7 waves
-// on a CU, about 1.5 per SIMD, for steps that pass through LDS twice, a division
+// on a CU, 1.75 per SIMD, for steps that pass through LDS twice, a division
 // and a root; FP64 issue is 180 us of the 64^3 HEXA8 mesh's 490 (1083 with
 // element matrices), its 0.52 GB store 60 us at the chip's copy rate.  Reference
 // gradients in LDS were 10 us slower, recomputing the node's own gradient in
@@ -93,9 +93,9 @@ int row_plan(int Nn, int dof_n, int nPe, const int* node_ptr, const int* node_co
   return check_launch("row_plan");
 }
 
-// LDS a block may use for its rows (the groups' 8 KB at most come on top): three
-// blocks on a CU.  Longer rows than this allows (HEXA8: 85 nodes, TETRA10: 170)
-// go through element matrices.
+// LDS a block may use for its rows (the groups' arrays, 0.9 to 6.2 KB, come on
+// top): three blocks on a CU, two of HEXA8.  Longer rows than this allows (HEXA8:
+// 85 nodes, TETRA10: 170) go through element matrices.
 constexpr size_t ASM_ROWS_MAX = 48 * 1024;
 
 struct AsmMesh {

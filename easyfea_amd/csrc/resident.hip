@@ -52,12 +52,13 @@
 //
 // What bounds it: the two exchanges (a store to memory and a load from it past
 // the L2s, about 1 us each way; 2,500 to 3,500 cycles for the halo, 3,000 for
-// the sums of 8 blocks, 5,800 of 256), then the block's own chain of LDS reads
+// the sums of 6 blocks, 5,800 of 256), then the block's own chain of LDS reads
 // and barriers.  Measured per iteration, the launch-per-step solve before and
-// this one: QUAD4 32^2 (8 blocks) 15.9 -> 4.8 us, 360 x 39 (64) 16.5 -> 5.6,
-// TRI3 251 x 249 (256) 22 -> 6.8, notched TRI3 200^2 (161) 20 -> 7.6, HEXA8
-// 30^3 (236) 42.6 -> 12.6, scalar QUAD4 700^2 (240) 28 -> 7.6, 1024^2 (229)
-// 50 -> 16; block Jacobi on 360 x 39 10.2 -> 4.0.
+// this one: QUAD4 32^2 (6 blocks) 15.9 -> 5.1 us, 360 x 39 (64) 16.5 -> 5.3,
+// TRI3 251 x 249 (256) 22 -> 6.6, notched TRI3 200^2 (161) 20 -> 8.0 and its
+// scalar system (80) 10.9 -> 4.2, HEXA8 30^3 (236) 42.6 -> 11.7, 31^3 (256)
+// 40 -> 12.0, scalar QUAD4 700^2 (240) 28 -> 6.0, 1024^2 (229) 50 -> 12.5;
+// block Jacobi on 360 x 39 10.2 -> 4.0.
 //
 // It replaces the same call as efea_solve_pcg: __Solver_1
 // (Simulations/Solvers.py:502-553) with _Solve_Axb's backends
