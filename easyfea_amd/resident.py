@@ -34,7 +34,8 @@ def shape(dof_n: int, max_neighbours: int, min_passes: int) -> Optional[tuple]:
 def bisect(coord: np.ndarray, parts: int) -> list:
     """The nodes in ``parts`` compact groups of nearly equal size (recursive
     coordinate bisection), each in increasing order."""
-    c = np.ascontiguousarray(coord, dtype=np.float64)
+    c = np.zeros((coord.shape[0], 3))
+    c[:, :coord.shape[1]] = coord  # of one to three columns
     order, ptr_ = np.empty(c.shape[0], dtype=np.int32), np.empty(parts + 1, dtype=np.int32)
     _lib.call("efea_resident_bisect", c.shape[0], c.ctypes.data, parts, order.ctypes.data, ptr_.ctypes.data)
     return np.split(order, ptr_[1:-1])
@@ -150,10 +151,10 @@ def collection(nm: int, nagg: int, pc: dict) -> np.ndarray:
 def neighbours(rows: torch.Tensor, node_ptr: torch.Tensor, node_cols: torch.Tensor, lanes: int, slots: int,
                passes: int) -> dict:
     """Halo lists, exchange numbers and the local neighbour positions of a
-    layout, as ``include/efea.h`` describes them (host tensors)."""
+    layout, as ``include/efea.h`` describes them, on the host."""
     nblk, nloc = rows.shape
     kept = slots - 1 if lanes == 1 else slots  # a scalar row's own node has no entry
-    rows, node_ptr, node_cols = (t.to(torch.int32).contiguous() for t in (rows, node_ptr, node_cols))
+    rows, node_ptr, node_cols = (t.to("cpu", torch.int32).contiguous() for t in (rows, node_ptr, node_cols))
     i32 = dict(dtype=torch.int32)
     out = dict(lidx=torch.empty(nblk * passes * kept * 64 * WAVES, dtype=torch.int16),
                halo_ptr=torch.empty(nblk + 1, **i32), halo_ex=torch.empty(node_cols.numel(), **i32),

@@ -147,6 +147,8 @@ def test_bisection_parts(n, parts):
     assert all((np.diff(p) > 0).all() and p.size <= -(-n // parts) for p in out)
     again = R.bisect(coord, parts)
     assert all(np.array_equal(a, b) for a, b in zip(out, again))
+    plane = R.bisect(np.asfortranarray(coord[:, :2]), parts)
+    assert sum(p.size for p in plane) == n
 
 
 def test_neighbours_refuses_rows_that_do_not_fit():
