@@ -950,6 +950,7 @@ class SolveJob:
             kind = "pcg2p"
         else:
             return None
+        PendingSolve.end_open()
         ws = ws or Workspace()
         self._prepare()
         if self.resident is None and not self.pipelined:  # a pause has begun since
@@ -963,7 +964,6 @@ class SolveJob:
         else:
             entry, args = kind, (self._pcgp_args if kind == "pcgp" else self._pcg2p_args)(ws, check_every, budget)
         s = stream_ptr()
-        PendingSolve.end_open()
         _lib.call(f"efea_{entry}_start", *args, s)
         return PendingSolve(self, ws, kind, args, s, entry)
 

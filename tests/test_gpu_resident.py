@@ -304,7 +304,8 @@ def test_a_start_ends_its_thread_s_open_one(mode, entry, monkeypatch):
         assert torch.equal(j.x, whole[k].x)
 
     jobs = [job(0, 3), job(1, 60)]
-    first, second = [j.start() for j in jobs]
+    ws = dv.Workspace()  # of both: the second, larger one takes another buffer
+    first, second = [j.start(ws) for j in jobs]
     assert first.entry == second.entry == entry
     for p in (second, first):
         check(jobs.index(p.job), p.job, p.finish())
