@@ -950,13 +950,13 @@ class SolveJob:
             kind = "pcg2p"
         else:
             return None
-        PendingSolve.end_open()
         ws = ws or Workspace()
         self._prepare()
         if self.resident is None and not self.pipelined:  # a pause has begun since
             return None
         if self.before_solve is not None and self.before_solve():
             self._redo_setup()
+        PendingSolve.end_open()  # before a shared workspace is asked for again
         check_every, _ = self._polls()
         budget = deferred_budget(self.expected_iterations, kind)
         if self.resident is not None:
